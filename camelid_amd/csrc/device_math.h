@@ -122,6 +122,29 @@ CM_HD float glibc_expf_t(float x, const uint64_t* tab) {
   return (float)y;
 }
 
+// The same for x <= 0 or NaN (a softmax exponent s - max), without branches: of the special cases
+// only -inf and the underflow below -0x1.9fe368p6 are left, both 0, and a NaN passes through the
+// evaluation.
+CM_HD float glibc_expf_nonpos_t(float x, const uint64_t* tab) {
+  const double kInvLn2N = 0x1.71547652b82fep+0 * 32.0;
+  const double kShift = 0x1.8p+52;
+  const double C0 = 0x1.c6af84b912394p-5 / (32.0 * 32.0 * 32.0);
+  const double C1 = 0x1.ebfce50fac4f3p-3 / (32.0 * 32.0);
+  const double C2 = 0x1.62e42ff0c52d6p-1 / 32.0;
+  const float xc = x < -0x1.9fe368p6f ? -0x1.9fe368p6f : x;
+  const double xd = (double)xc;
+  double kd = fma(kInvLn2N, xd, kShift);
+  const uint64_t ki = d2u(kd);
+  kd -= kShift;
+  const double r = fma(kInvLn2N, xd, -kd);
+  const double sc = u2d(tab[ki & 31u] + (ki << 47));
+  const double z = fma(C0, r, C1);
+  double y = fma(C2, r, 1.0);
+  y = fma(z, r * r, y);
+  y = y * sc;
+  return x < -0x1.9fe368p6f ? 0.0f : (float)y;
+}
+
 CM_HD float glibc_expf(float x) { return glibc_expf_t(x, kExp2Tab); }
 
 // Q8_0 block quantizer (inference.rs:16953-16971): amax fold, scale = f16(amax/127),

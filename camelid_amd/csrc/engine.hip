@@ -190,10 +190,10 @@ struct camelid_hip_engine {
   int8_t* pf_kq = nullptr;
   int8_t* pf_kqt = nullptr;  // the chunk's Q8_K quants in the class-major order of the Q6_K GEMM
   int32_t* pf_kbs = nullptr;
-  // score rows of the tiled prefill attention (cm::k_attn_prefill_tile; CAMELID_HIP_ATT_TILE=0:
+  // score rows of the tiled prefill attention (cm::k_attn_prefill_mm; CAMELID_HIP_ATT_TILE=0:
   // one workgroup per (head, token) instead), sized for a chunk ending at max_pos
   bool att_tile = true;
-  uint32_t att_tile_pos = 1024;  // chunks ending below this position: per-token kernel (CAMELID_HIP_ATT_TILE_POS)
+  uint32_t att_tile_pos = 0;  // chunks ending below this position: per-token kernel (CAMELID_HIP_ATT_TILE_POS)
   float* pf_sc = nullptr;
   // verify scratch (allocated on first use): inputs of up to CAMELID_MAX_VERIFY_K tokens,
   // their logits and greedy tokens
@@ -1365,13 +1365,6 @@ void run_embed(camelid_hip_engine* e) {
 // ---------------------------------------------------------------- batched prefill
 constexpr uint32_t PREFILL_CHUNK = 512;  // tokens per pass over the layers
 
-// Scratch floats the tiled prefill attention needs for T tokens up to position pos0 + T - 1
-// (its score rows: 64 per tile, one tile per TQ tokens of each KV head).
-size_t attn_prefill_scratch(uint32_t n_heads, uint32_t n_kv, uint32_t T, uint32_t pos_end) {
-  const uint32_t tq = (uint32_t)cm::apt_tq((int)(n_heads / n_kv));
-  return (size_t)n_kv * ((T + tq - 1) / tq) * cm::APT_R * cm::apt_pitch(pos_end);
-}
-
 int ensure_prefill_buffers(camelid_hip_engine* e) {
   if (e->pf_h) return 0;
   const camelid_hip_dims& d = e->d;
@@ -1382,8 +1375,8 @@ int ensure_prefill_buffers(camelid_hip_engine* e) {
       dev_alloc(e, &e->pf_q, tc * nq) || dev_alloc(e, &e->pf_gu, tc * 2 * d.ffn_dim) ||
       dev_alloc(e, &e->pf_xq, tc * act) || dev_alloc(e, &e->pf_xs, tc * act / 32))
     return 1;
-  if (e->att_tile && cm::apt_hd_ok((int)d.head_dim) && d.n_heads / d.n_kv_heads <= (uint32_t)cm::APT_R &&
-      dev_alloc(e, &e->pf_sc, attn_prefill_scratch(d.n_heads, d.n_kv_heads, PREFILL_CHUNK, e->kvs)))
+  if (e->att_tile && cm::apm_hd_ok((int)d.head_dim) &&
+      dev_alloc(e, &e->pf_sc, cm::apm_scratch((int)d.n_heads, (int)d.n_kv_heads, (int)PREFILL_CHUNK, e->kvs)))
     return 1;
   if (!e->any_kquant) return 0;
   return dev_alloc(e, &e->pf_kd, tc * act / 256) || dev_alloc(e, &e->pf_kq, tc * act) ||
@@ -1513,40 +1506,33 @@ int q8_scan_inf_scales(Q8Mat* m, hipStream_t s) {
   return 0;
 }
 
-// Causal attention of a prefill chunk: the tiled kernel (K/V rows shared by a tile of query
-// tokens and the heads of their KV group) when scratch is given, the geometry has it and the
-// chunk has at least tile_min tokens and reaches position tile_pos, else one workgroup per
-// (head, token): a verify batch of a few tokens spreads wider that way, and below ~1K positions
-// the per-token kernel measured faster (C5 1023-token prefill 0.072 vs 0.076 s, C3 511 tokens
-// 0.016 vs 0.018 s; C4 8191 tokens 1.52 -> 1.03 s tiled).
-constexpr uint32_t APT_TILE_MIN = 32;
-constexpr uint32_t APT_TILE_POS = 1024;
+// Whether the tiled attention of a prefill chunk (cm::k_attn_prefill_mm: 16 rows of a KV head per
+// workgroup) is faster than one workgroup per (head, token) (cm::k_attn_prefill).  The per-token
+// kernel does about 32,000 (head, token, position) terms of 128 dims per us over the whole device;
+// a tile's time is its own latency, about 6 us + 0.072 us per position, as long as the device
+// holds all tiles at once, and about half the per-token kernel's time per term beyond.  Measured
+// (us, per token / tiled): 24 heads of 128 dims, 511 tokens 96 / 62, 32 tokens at 2000 positions
+// 54 / 147, 16 at 300 12 / 31; 32 heads of 64 dims, 127 tokens 12 / 17.
+bool attn_prefill_tiled(uint32_t hd, uint32_t n_heads, uint32_t T, uint32_t pos0) {
+  if (!cm::apm_hd_ok((int)hd)) return false;
+  const double pos = pos0 + 0.5 * T, terms = (double)T * n_heads * pos * hd / 128.0;
+  return terms > 32000.0 * (3.0 + 0.075 * ((double)pos0 + T));
+}
+
+// Causal attention of a prefill chunk: tiled when scratch (cm::apm_scratch floats) is given, else
+// one workgroup per (head, token).
 void launch_attn_prefill(uint32_t hd, uint32_t n_heads, uint32_t n_kv, uint32_t T, const float* q, const uint16_t* kc,
                          const uint16_t* vc, int layer, int kvs, int pos0, float scale, float* att, int8_t* xq, float* xs,
-                         hipStream_t s, float* scratch = nullptr, uint32_t tile_min = APT_TILE_MIN,
-                         uint32_t tile_pos = APT_TILE_POS) {
-  if (scratch && cm::apt_hd_ok((int)hd) && n_heads / n_kv <= (uint32_t)cm::APT_R && T >= tile_min &&
-      (uint32_t)pos0 + T >= tile_pos) {
-    const uint32_t tq = (uint32_t)cm::apt_tq((int)(n_heads / n_kv));
-    const size_t pitch = cm::apt_pitch((size_t)pos0 + T);
-    const dim3 grid(n_kv, (T + tq - 1) / tq);
-    // 1024 threads (2 rows per thread, 110 VGPRs: four waves per SIMD) by default; 512 (4 rows
-    // per thread, 155 VGPRs, two waves per SIMD) with CAMELID_HIP_APT_NT=512.  C4's 8191-token
-    // prefill: 1.004 s at 512, 0.915 s at 1024 (a single wave issues one VALU instruction per
-    // ~7 clocks, so two waves leave a SIMD idle between their issues)
-    const char* nt = std::getenv("CAMELID_HIP_APT_NT");
-    const bool wide = !(nt && std::atoi(nt) == 512);
-#define CM_APT(HD, NT)                                                                                        \
-  CM_LAUNCH((cm::k_attn_prefill_tile<HD, NT>), grid, dim3(NT), cm::apt_lds_bytes(HD), s, q, (int)n_heads,     \
-            (int)n_kv, kc, vc, layer, kvs, pos0, (int)T, scale, scratch, pitch, att, xq, xs)
-    if (hd == 64) {
-      if (wide) CM_APT(64, 1024);
-      else CM_APT(64, 512);
-    } else {
-      if (wide) CM_APT(128, 1024);
-      else CM_APT(128, 512);
-    }
-#undef CM_APT
+                         hipStream_t s, float* scratch) {
+  if (scratch) {
+    const dim3 grid(n_kv * (uint32_t)cm::apm_tiles((int)(n_heads / n_kv), (int)T));
+    const size_t pitch = cm::apm_pitch((size_t)pos0 + T);
+#define CM_APM(HD)                                                                                               \
+  CM_LAUNCH(cm::k_attn_prefill_mm<HD>, grid, dim3(cm::apm_nt(HD)), 0, s, q, (int)n_heads, (int)n_kv, kc, vc, layer, \
+            kvs, pos0, (int)T, scale, scratch, pitch, att, xq, xs)
+    if (hd == 64) CM_APM(64);
+    else CM_APM(128);
+#undef CM_APM
     return;
   }
   const size_t lds = (((size_t)pos0 + T + 3) & ~(size_t)3) * 4;
@@ -1557,6 +1543,11 @@ void launch_attn_prefill(uint32_t hd, uint32_t n_heads, uint32_t n_kv, uint32_t 
   else if (hd == 128) CM_AP(128);
   else CM_AP(256);
 #undef CM_AP
+}
+
+// The scratch of a chunk that runs the tiled attention, else null.
+float* pf_scratch(const camelid_hip_engine* e, uint32_t T, uint32_t pos0) {
+  return pos0 + T >= e->att_tile_pos && attn_prefill_tiled(e->d.head_dim, e->d.n_heads, T, pos0) ? e->pf_sc : nullptr;
 }
 
 // One chunk of T prompt tokens at positions pos0.. through every layer; the residual rows
@@ -1596,7 +1587,7 @@ void prefill_layer_generic(camelid_hip_engine* e, uint32_t l, const float* cosv,
             L.k_norm, d.eps, e->pf_q, e->kc, e->vc, (int)l, (int)e->kvs, (const uint32_t*)nullptr, (int)pos0,
             (int)half);
   launch_attn_prefill(d.head_dim, d.n_heads, d.n_kv_heads, T, e->pf_q, e->kc, e->vc, (int)l, (int)e->kvs, (int)pos0,
-                      scale, e->pf_att, e->pf_xq, e->pf_xs, s, e->pf_sc, APT_TILE_MIN, e->att_tile_pos);
+                      scale, e->pf_att, e->pf_xq, e->pf_xs, s, pf_scratch(e, T, pos0));
   if (L.p[3].quant != CAMELID_Q8_0)
     CM_LAUNCH(cm::k_quantize_q8k, dim3(T * nq / 256), dim3(256), 0, s, e->pf_att, e->pf_kd, e->pf_kq,
               e->pf_kbs);
@@ -1635,7 +1626,7 @@ void prefill_chunk(camelid_hip_engine* e, const float* cosv, const float* sinv, 
               L.k_norm, d.eps, e->pf_q, e->kc, e->vc, (int)l, (int)e->kvs, (const uint32_t*)nullptr, (int)pos0,
               (int)half);
     launch_attn_prefill(d.head_dim, d.n_heads, d.n_kv_heads, T, e->pf_q, e->kc, e->vc, (int)l, (int)e->kvs,
-                        (int)pos0, scale, nullptr, e->pf_xq, e->pf_xs, s, e->pf_sc, APT_TILE_MIN, e->att_tile_pos);
+                        (int)pos0, scale, nullptr, e->pf_xq, e->pf_xs, s, pf_scratch(e, T, pos0));
     gemm(L.o, e->pf_h, e->pf_h);
     launch_rmsnorm_quant(e->pf_h, L.ffn_norm, d.hidden, d.eps, e->pf_xq, e->pf_xs, nullptr, s, cm::Prefetch{}, T);
     gemm(L.gu, e->pf_gu, nullptr);
@@ -2784,15 +2775,15 @@ int camelid_hip_attention_prefill(const float* qrot, const uint16_t* kc, const u
   if (max_pos % 8) return fail(nullptr, "the KV position stride (max_pos) must be a multiple of 8");
   if (tokens == 0 || (size_t)pos0 + tokens > max_pos) return fail(nullptr, "positions beyond max_pos");
   if (((size_t)pos0 + tokens) * 4 > 64 * 1024) return fail(nullptr, "more than 16384 positions");
-  // the tiled kernel whenever it applies (any token count), unless CAMELID_HIP_ATT_TILE=0;
-  // its score scratch is allocated for the call
+  // CAMELID_HIP_ATT_TILE: 1 the tiled kernel wherever it applies, 0 never, else by size; its score
+  // scratch is allocated for the call
   const char* te = std::getenv("CAMELID_HIP_ATT_TILE");
-  const bool tiled = !(te && std::atoi(te) == 0) && cm::apt_hd_ok((int)hd) && n_heads / n_kv <= (uint32_t)cm::APT_R;
+  const bool tiled = te ? std::atoi(te) != 0 && cm::apm_hd_ok((int)hd) : attn_prefill_tiled(hd, n_heads, tokens, pos0);
   float* scratch = nullptr;
-  if (tiled && hipMalloc(&scratch, attn_prefill_scratch(n_heads, n_kv, tokens, pos0 + tokens) * 4) != hipSuccess)
+  if (tiled && hipMalloc(&scratch, cm::apm_scratch((int)n_heads, (int)n_kv, (int)tokens, (size_t)pos0 + tokens) * 4) != hipSuccess)
     return fail(nullptr, "scratch allocation failed");
   launch_attn_prefill(hd, n_heads, n_kv, tokens, qrot, kc, vc, (int)layer, (int)max_pos, (int)pos0, scale, att_out,
-                      xq, xs, (hipStream_t)stream, scratch, 1, 0);
+                      xq, xs, (hipStream_t)stream, scratch);
   if (scratch) {
     const hipError_t st = hipStreamSynchronize((hipStream_t)stream);
     (void)hipFree(scratch);

@@ -6,7 +6,8 @@
 //   RMSNorm rows     k_rmsnorm_quant with gridDim.y = T (one workgroup per token)
 //   projections      k_gemm_q8: int8 matrix cores for the per-block dots, f32 folds in block order
 //   QK-norm/RoPE/KV  k_rope_kv with gridDim.y = T
-//   attention        k_attn_prefill: one workgroup per (head, token), causal over [0, pos]
+//   attention        k_attn_prefill_mm: 16 (head, token) rows per workgroup, products on the matrix
+//                    cores; k_attn_prefill: one workgroup per (head, token); causal over [0, pos]
 //   SwiGLU           k_silu_rows
 #pragma once
 #include "kernels_decode.h"
@@ -556,329 +557,311 @@ __global__ __launch_bounds__(AP_NT) void k_attn_prefill(const float* __restrict_
 
 // ---------------------------------------------------------------------------
 // Causal attention of a prefill chunk, tiled over query tokens (attention_batched and the
-// flash prefill of cuda_resident.rs:1994, :2523-2757; CPU inference.rs:23945-24025 per token).
-// One workgroup per (KV head g, tile of TQ consecutive tokens).  Its rows are the (query head
-// g*rep + i, token t0 + j) pairs, row r = i*TQ + j, at most 64 of them, so each K and V row of
-// the cache is loaded once per tile and used by every row of it (k_attn_prefill loads it once
-// per (head, token)).  Each row's arithmetic is k_attn_prefill's, in the same order:
-//   A  scores s_p = (sum_d q_d * k_pd, d in order) * scale over 128-position blocks of K
-//      granules in LDS, 4 rows x 4 positions per thread (16 independent chains); the scores go
-//      to the scratch rows sc[r][p]; the row maximum (exact, any order);
-//   B  e_p = expf(s_p - m_r), written back over the score, and folded into the row's sum in
-//      position order by one lane per row (wave 0); inv_r = 1 / sum;
-//   C  prob_p = e_p * inv_r, out_rd = fold_p prob_p * v_pd in position order: the block's V
-//      granules in LDS, 4 rows x DB dims per thread.
-// Every thread reads back only the scratch words it wrote itself (phases A, B and C share one
-// (rows, positions) assignment), so no cache line of another thread's is ever stale.  The next
-// block's global loads (K and V granules, scratch words) go out before the current block is
-// computed.  A row's positions p >= P_r = pos0 + t + 1 contribute e = 0 to its sum and nothing
-// to its outputs (masked adds in the blocks that reach past the tile's first row); a sum that
-// starts at +0 and adds non-negative terms is never -0, so adding +0 leaves it unchanged.  A
-// row with P_r = 1 copies the V row (inference.rs:23564-23575).  Outputs as k_attn_prefill:
-// f32 rows (optional) and Q8_0 per 32-value block.  Scratch: sc + tile_index * 64 * pitch
-// floats, pitch >= P_max rounded up to 128.  Dynamic LDS: apt_lds_bytes(HD).
-constexpr int APT_NT = 1024;  // threads (the kernel is also instantiated at 512)
-constexpr int APT_R = 64;    // rows per tile
-constexpr int APT_PB = 128;  // positions per block
-constexpr int APT_ES = APT_PB + 4;  // row stride of the exponential / probability block
-__host__ __device__ constexpr int apt_tq(int rep) { return rep >= APT_R ? 1 : APT_R / rep; }
-__host__ __device__ constexpr size_t apt_pitch(size_t pmax) { return (pmax + APT_PB - 1) / APT_PB * APT_PB; }
-__host__ __device__ constexpr size_t apt_lds_bytes(int hd) {
-  return (size_t)hd * APT_R * 4 + (size_t)(hd / 8) * APT_PB * 16 + (size_t)APT_R * APT_ES * 4;
+// flash prefill of cuda_resident.rs:1994, :2523-2757; CPU inference.rs:23945-24025 per token),
+// its products formed on the matrix cores.
+// Both sums of the attention are, per term, an outer product: term d of the scores of 16 rows
+// and some positions is q_d[row] * k_d[position], term p of the outputs of 16 rows and some dims
+// is prob_p[row] * v_p[dim].  v_mfma_f32_16x16x1_4b with a zero addend forms four such 16 x 16
+// product tiles, each product rounded once to nearest even (bit for bit v_mul_f32, subnormals
+// included), and the VALU then only adds, in order.  1024 products and their adds take 67-77
+// clocks of a SIMD (two or more waves, four product tiles issued together) where products from
+// v_fma_mix_f32 (half the rate of v_add_f32) and their adds take 111, and the operands are one
+// register each instead of LDS reads of both.
+//
+// One workgroup per (16 rows, KV head), the KV heads of a tile in consecutive workgroups (with 8 of
+// them, a head's K/V stay in one XCD's L2): row R = 16 * tile + r of the KV head's T * rep rows is
+// query head R % rep of the group at token R / rep.  W = HD / 32 waves; lane l of a wave is
+// l % 16 = lr in block l / 16 = lb.  A wave's product covers 16 rows x 32 columns (positions or
+// dims) for two terms: blocks 0, 1 are columns 0-15, 16-31 of the first term, blocks 2, 3 of the
+// second (cbsz 1: blocks 0, 1 share one A block, 2, 3 another; abid picks which of two terms'
+// rows a register holds for each).  A term pair is (8 g + c, 8 g + 4 + c): four products c = 0..3
+// give the 8 terms of one 16-byte granule, which the adds take in order.
+//   A  wave w takes the 32-position blocks w, w + W, ...: q in HD / 4 registers, K straight from
+//      global memory (8 bytes of a granule per lane); the scores (acc * scale) go to the scratch,
+//      cells [row quad][position][4 rows], the row maxima (exact, any order) to LDS;
+//   B  wave w takes 16 / W rows: e_p = expf(s_p - m_r), folded in position order by one lane per
+//      row, and written over the scores with every 4 x 4 cell transposed;
+//   C  wave w takes dims 32 w ..: prob_p = e_p * inv_r (one 16-byte load per lane and 16
+//      positions, already the A operand's layout), V straight from global memory.
+// Each row's arithmetic and order are k_attn_prefill's.  Positions p >= P_r contribute e = 0 to
+// the sum (a non-negative sum from +0 is never -0, so +0 leaves it unchanged) and are not added
+// to the outputs (selects where a row of the tile ends).  A row with P_r = 1 copies the V row
+// (inference.rs:23564-23575).  Outputs as k_attn_prefill: f32 rows (optional) and Q8_0 per
+// 32-value block.
+// Bound by the adds and the f32 matrix issue, which share the f32 units and so do not overlap, and
+// by the scratch (20 bytes per row and position) at 8K positions.  Measured (32 heads of 128 dims,
+// 511-512 tokens): 72 us at positions 0.., 173 us at 512.., 746 us at 3584.., 1435 us at 7680..,
+// where one workgroup per (head, token) takes 128, 319, 1625 and 4036 us and the same tiling with
+// v_fma_mix products (64 rows per 1024-thread workgroup, operands in LDS) took 1281 us on average
+// over the chunks of an 8191-token prompt (740 us now).
+constexpr int APM_R = 16;   // rows per tile
+constexpr int APM_PB = 64;  // the scratch's positions are padded to this
+__host__ __device__ constexpr int apm_tiles(int rep, int T) { return (T * rep + APM_R - 1) / APM_R; }
+__host__ __device__ constexpr size_t apm_pitch(size_t pmax) { return (pmax + APM_PB - 1) / APM_PB * APM_PB; }
+__host__ __device__ constexpr bool apm_hd_ok(int hd) { return hd == 64 || hd == 128; }
+// threads per workgroup
+__host__ __device__ constexpr int apm_nt(int hd) { return hd * 2; }
+// scratch floats for T tokens up to position pos_end - 1
+__host__ __device__ constexpr size_t apm_scratch(int n_heads, int n_kv, int T, size_t pos_end) {
+  return (size_t)n_kv * apm_tiles(n_heads / n_kv, T) * APM_R * apm_pitch(pos_end);
 }
-__host__ __device__ constexpr bool apt_hd_ok(int hd) { return hd == 64 || hd == 128; }
 
-// the f16 value e of the 8 in a 16-byte granule times x, rounded once (v_fma_mix)
-__device__ __forceinline__ float mul_gran(float x, const uint4& g, int e) {
-  const uint32_t w = e < 2 ? g.x : e < 4 ? g.y : e < 6 ? g.z : g.w;
-  return (e & 1) ? mul_f16_hi(x, w) : mul_f16_lo(x, w);
+typedef float v16f_t __attribute__((ext_vector_type(16)));
+
+// element 4 b + i of lane l: a[row 4 (l / 16) + i, held in block 2 (b / 2) + AB] * b[lane 16 b + l % 16]
+template <int AB>
+__device__ __forceinline__ v16f_t outer16x2(float a, float b) {
+  const v16f_t z = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, z, 1, AB, 0);
 }
 
-template <int HD, int NT = APT_NT>
-__global__ __launch_bounds__(NT) void k_attn_prefill_tile(
+// The f32 of the f16 in either half of w.  The conversions are left to the compiler, which knows
+// the wait states a matrix instruction needs after its operand is written; the shift is opaque
+// to it so that the high half takes a shift and a plain conversion (7 clocks) and not one with a
+// sub-word select (about 10).
+__device__ __forceinline__ float half_lo(uint32_t w) { return half_bits_to_float((uint16_t)w); }
+__device__ __forceinline__ float half_hi(uint32_t w) {
+  uint32_t h;
+  asm("v_lshrrev_b32 %0, 16, %1" : "=v"(h) : "v"(w));
+  return half_bits_to_float((uint16_t)h);
+}
+
+// acc[j] (j = 4 * column block + row) += the 8 terms of a granule, in order: a[c] holds the rows'
+// factors of terms c and 4 + c, f the columns' (two f16 pairs per lane: terms 0-3 in the lanes of
+// blocks 0, 1, terms 4-7 in those of blocks 2, 3).  MASK: term e is added where e < left[j % 4].
+template <int AB, bool MASK>
+__device__ __forceinline__ void outer_terms(float (&acc)[8], const float* a, const uint2& f, const int* left) {
+  const v16f_t t0 = outer16x2<AB>(a[0], half_lo(f.x)), t1 = outer16x2<AB>(a[1], half_hi(f.x));
+  const v16f_t t2 = outer16x2<AB>(a[2], half_lo(f.y)), t3 = outer16x2<AB>(a[3], half_hi(f.y));
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const v16f_t& t = c == 0 ? t0 : c == 1 ? t1 : c == 2 ? t2 : t3;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        acc[j] = !MASK || 4 * h + c < left[j & 3] ? acc[j] + t[8 * h + j] : acc[j];
+    }
+  }
+}
+
+template <int HD>
+__global__ __launch_bounds__(HD * 2, 4) void k_attn_prefill_mm(
     const float* __restrict__ qrot, int n_heads, int n_kv, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, int layer, int kvs, int pos0, int T, float scale, float* __restrict__ scg,
     size_t pitch, float* __restrict__ att_out, int8_t* __restrict__ xq, float* __restrict__ xs) {
-  static_assert(apt_hd_ok(HD), "tiled prefill attention: head_dim 64 or 128");
-  constexpr int R8 = HD / 8;            // K granules per position
-  constexpr int DB = HD / 32;           // output dims per thread in phase C (32 dim groups)
-  constexpr int KG = R8 * APT_PB;       // K granules of a block (as many V granules: APT_PB/8 x HD)
-  constexpr int GPT = KG / NT;          // of them per thread
-  constexpr int NRG = NT / 32;          // row groups: 32 threads each (4 positions / DB dims a thread)
-  constexpr int RPT = APT_R / NRG;      // rows per thread: 4 at 512 threads, 2 at 1024
-  static_assert(KG == (APT_PB / 8) * HD && KG % NT == 0 && (RPT == 2 || RPT == 4), "block staging");
-  extern __shared__ __align__(16) float4 dyn[];
-  float* qs = reinterpret_cast<float*>(dyn);              // [HD][64] q tile; later out rows [64][HD]
-  uint4* kb = reinterpret_cast<uint4*>(qs + HD * APT_R);  // K granules [R8][PB], then V [PB/8][HD]
-  float* eb = reinterpret_cast<float*>(kb + KG);          // [64][APT_ES] exponentials / probabilities
-  __shared__ float mrow[APT_R], irow[APT_R];
-  __shared__ int prow[APT_R];  // P_r (0: no row in this slot)
-  const int tid = threadIdx.x;
-  const int rep = n_heads / n_kv, TQ = apt_tq(rep);
-  const int g = blockIdx.x, ntile = gridDim.y, tile = ntile - 1 - (int)blockIdx.y;  // longest first
-  const int t0 = tile * TQ;
-  const size_t hbase = kv_head_base(layer, n_kv, g, HD, kvs);
-  const uint4* kg = reinterpret_cast<const uint4*>(kc + hbase);
-  const uint4* vg = reinterpret_cast<const uint4*>(vc + hbase);
-  float* sc = scg + ((size_t)g * ntile + tile) * APT_R * pitch;
-  auto row_head = [&](int r) { return g * rep + r / TQ; };
-  auto row_tok = [&](int r) { return t0 + r % TQ; };
-  if (tid < APT_R) {
-    const int i = tid / TQ, t = t0 + tid % TQ;
-    prow[tid] = (i < rep && t < T) ? pos0 + t + 1 : 0;
-  }
-  const int pmax = pos0 + min(t0 + TQ, T);  // the tile's longest row
-  const int pmin = pos0 + t0 + 1;           // its shortest
-  const int nblk = (pmax + APT_PB - 1) / APT_PB;
-  // staging of block b through registers: K granule (u, p) or V granule (group, d) number
-  // i = tid + NT * k (GPT = 1, 2 or 4 named registers: an array here went to scratch memory)
-  const int glast = (pmax - 1) >> 3;
-  uint4 stg0, stg1, stg2, stg3;
-  auto kgran = [&](int b, int k) {
-    const int i = tid + NT * k, u = i / APT_PB, p = i % APT_PB;
-    return kg[(size_t)u * kvs + min(b * APT_PB + p, pmax - 1)];
+  static_assert(apm_hd_ok(HD), "tiled prefill attention: head_dim 64 or 128");
+  constexpr int W = HD / 32;              // waves
+  constexpr int RW = APM_R / W;           // rows per wave in phase B
+  constexpr int LP = RW / 4;              // lanes per position there (4 rows each)
+  constexpr int PS = 64 / LP;             // positions per step there
+  constexpr int ES = PS + 4;              // row stride of its LDS block
+  constexpr int NM = HD / 16;             // 16-dim stages of a score
+  __shared__ __align__(16) float eb[W][RW * ES];
+  __shared__ float smax[W][APM_R], sinv[APM_R];
+  __shared__ __align__(16) float os[APM_R][HD + 4];
+  __shared__ uint64_t etab[32];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int lr = lane & 15, lb = lane >> 4;
+  const int rep = n_heads / n_kv, ntile = apm_tiles(rep, T);
+  const int kvh = (int)blockIdx.x % n_kv, tile = ntile - 1 - (int)blockIdx.x / n_kv;  // longest first
+  const int R0 = tile * APM_R, nr = min(APM_R, T * rep - R0);           // its rows
+  const size_t hbase = kv_head_base(layer, n_kv, kvh, HD, kvs);
+  const uint2* kg = reinterpret_cast<const uint2*>(kc + hbase);
+  const uint2* vg = reinterpret_cast<const uint2*>(vc + hbase);
+  float* sc = scg + ((size_t)kvh * ntile + tile) * APM_R * pitch;
+  auto row_off = [&](int r) {  // element offset of row r in the [T][n_heads * HD] arrays
+    const int R = R0 + min(r, nr - 1);  // (rows past the last repeat it and are not stored)
+    return (size_t)(R / rep) * n_heads * HD + (size_t)(kvh * rep + R % rep) * HD;
   };
-  auto vgran = [&](int b, int k) {
-    const int i = tid + NT * k, gq = i / HD, d = i % HD;
-    return vg[(size_t)min(b * (APT_PB / 8) + gq, glast) * HD + d];
-  };
-#define APT_LOAD_K(b)                                       \
-  stg0 = kgran((b), 0);                                     \
-  if (GPT > 1) stg1 = kgran((b), 1);                        \
-  if (GPT > 2) {                                            \
-    stg2 = kgran((b), 2);                                   \
-    stg3 = kgran((b), 3);                                   \
-  }
-#define APT_LOAD_V(b)                                       \
-  stg0 = vgran((b), 0);                                     \
-  if (GPT > 1) stg1 = vgran((b), 1);                        \
-  if (GPT > 2) {                                            \
-    stg2 = vgran((b), 2);                                   \
-    stg3 = vgran((b), 3);                                   \
-  }
-#define APT_PUT()                                           \
-  kb[tid] = stg0;                                           \
-  if (GPT > 1) kb[tid + NT] = stg1;                         \
-  if (GPT > 2) {                                            \
-    kb[tid + 2 * NT] = stg2;                                \
-    kb[tid + 3 * NT] = stg3;                                \
-  }
-  static_assert(GPT == 1 || GPT == 2 || GPT == 4, "staging registers");
-  APT_LOAD_K(0)
-  // the q tile, transposed: qs[d][r]
-  for (int i = tid; i < APT_R * HD; i += NT) {
-    const int r = i / HD, d = i % HD;
-    const int t = row_tok(r);
-    const bool ok = r / TQ < rep && t < T;
-    qs[d * APT_R + r] = ok ? qrot[(size_t)t * n_heads * HD + (size_t)row_head(r) * HD + d] : 0.0f;
-  }
-  APT_PUT()
-  __syncthreads();
-  const int rg = tid >> 5, pg = tid & 31;  // rows RPT rg .. +RPT-1, block positions 4pg .. 4pg+3
-  int pr[RPT];
+  auto row_p = [&](int r) { return pos0 + (R0 + min(r, nr - 1)) / rep + 1; };  // P_r
+  const int pmax = row_p(nr - 1), pmin = row_p(0);
+  int pr[4];  // P of rows 4 lb + i, whose values this lane holds in a product
 #pragma unroll
-  for (int i = 0; i < RPT; ++i) pr[i] = prow[RPT * rg + i];
-  auto scw = [&](int i, int b) { return reinterpret_cast<float4*>(sc + (size_t)(RPT * rg + i) * pitch + b * APT_PB) + pg; };
-  // the q values of this thread's RPT rows for dim d (one LDS read)
-  auto qrows = [&](int d, float (&qv)[RPT]) {
-    if constexpr (RPT == 4) {
-      const float4 q4 = reinterpret_cast<const float4*>(qs + d * APT_R)[rg];
-      qv[0] = q4.x;
-      qv[1] = q4.y;
-      qv[2] = q4.z;
-      qv[3] = q4.w;
-    } else {
-      const float2 q2 = reinterpret_cast<const float2*>(qs + d * APT_R)[rg];
-      qv[0] = q2.x;
-      qv[1] = q2.y;
-    }
-  };
+  for (int i = 0; i < 4; ++i) pr[i] = row_p(4 * lb + i);
+  if (tid < 32) etab[tid] = kExp2Tab[tid];
+
   // ---- A: scores and row maxima
-  float rmax[RPT];
+  {
+    // q of row lr: register 4 m + c holds, in block b, dim 16 m + 8 (b % 2) + 4 (b / 2) + c
+    float q[4 * NM];
+    const float* qp = qrot + row_off(lr) + 8 * (lb & 1) + 4 * (lb >> 1);
 #pragma unroll
-  for (int i = 0; i < RPT; ++i) rmax[i] = -INFINITY;
-  for (int b = 0; b < nblk; ++b) {
-    if (b + 1 < nblk) {
-      APT_LOAD_K(b + 1)
+    for (int m = 0; m < NM; ++m) {
+      const float4 v = *reinterpret_cast<const float4*>(qp + 16 * m);
+      q[4 * m] = v.x;
+      q[4 * m + 1] = v.y;
+      q[4 * m + 2] = v.z;
+      q[4 * m + 3] = v.w;
     }
-    float acc[RPT][4];
+    float rm[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    const int nblk = (pmax + 31) / 32;
+    // this lane's halves of the K granules of a 16-dim stage, loaded KD stages ahead of their use
+    constexpr int KD = 1;
+    static_assert(NM % (KD + 1) == 0, "K ring");
+    uint2 kr[KD + 1][2];
+    auto kload = [&](uint2 (&r)[2], int b, int m) __attribute__((always_inline)) {
+      const int p = min(b * 32 + 16 * (lb & 1) + lr, pmax - 1);
+      const uint2* a = kg + ((size_t)(2 * m) * kvs + p) * 2 + (lb >> 1);
+      r[0] = a[0];
+      r[1] = a[2 * (size_t)kvs];
+    };
 #pragma unroll
-    for (int i = 0; i < RPT; ++i)
+    for (int m = 0; m < KD; ++m) kload(kr[m], min(wave, nblk - 1), m);
+    for (int b = wave; b < nblk; b += W) {
+      const int bn = min(b + W, nblk - 1);  // (the last block loads itself again)
+      float acc[8];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
-    for (int u = 0; u < R8; ++u) {
-      uint4 k4[4];
+      for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) k4[j] = kb[u * APT_PB + 4 * pg + j];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        float qv[RPT];
-        qrows(8 * u + e, qv);
-#pragma unroll
-        for (int i = 0; i < RPT; ++i)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc[i][j] += mul_gran(qv[i], k4[j], e);
+      for (int m = 0; m < NM; ++m) {
+        kload(kr[(m + KD) % (KD + 1)], m + KD < NM ? b : bn, (m + KD) % NM);
+        outer_terms<0, false>(acc, q + 4 * m, kr[m % (KD + 1)][0], nullptr);
+        outer_terms<1, false>(acc, q + 4 * m, kr[m % (KD + 1)][1], nullptr);
       }
-    }
-    const int p0 = b * APT_PB + 4 * pg;
 #pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-      float sv[4];
+      for (int u = 0; u < 2; ++u) {
+        const int p = b * 32 + 16 * u + lr;
+        float s[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        sv[j] = acc[i][j] * scale;
-        if (p0 + j < pr[i]) rmax[i] = fmaxf(rmax[i], sv[j]);
-      }
-      if (pr[i] > p0) *scw(i, b) = make_float4(sv[0], sv[1], sv[2], sv[3]);
-    }
-    __syncthreads();  // every wave is done with this block's K
-    if (b + 1 < nblk) {
-      APT_PUT()
-    }
-    __syncthreads();
-  }
-  APT_LOAD_V(0)  // (the first V block streams during the softmax)
-  // row maxima over the 32 threads of a row group (lanes 32 rg' .. 32 rg' + 31 of a wave)
-#pragma unroll
-  for (int i = 0; i < RPT; ++i) {
-#pragma unroll
-    for (int o = 16; o >= 1; o >>= 1) rmax[i] = fmaxf(rmax[i], __shfl_xor(rmax[i], o));
-    if (pg == 0) mrow[RPT * rg + i] = rmax[i];
-  }
-  __syncthreads();
-  float m[RPT];
-#pragma unroll
-  for (int i = 0; i < RPT; ++i) m[i] = mrow[RPT * rg + i];
-  // ---- B: exponentials (over the scores in the scratch), each row's sum in position order
-  float sum = 0.0f;
-  float4 snext[RPT];
-#pragma unroll
-  for (int i = 0; i < RPT; ++i) snext[i] = pr[i] > 4 * pg ? *scw(i, 0) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  for (int b = 0; b < nblk; ++b) {
-    const int p0 = b * APT_PB + 4 * pg;
-    float4 scur[RPT];
-#pragma unroll
-    for (int i = 0; i < RPT; ++i) scur[i] = snext[i];
-    if (b + 1 < nblk) {
-#pragma unroll
-      for (int i = 0; i < RPT; ++i) snext[i] = pr[i] > p0 + APT_PB ? *scw(i, b + 1) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
-#pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-      const float sv[4] = {scur[i].x, scur[i].y, scur[i].z, scur[i].w};
-      float ev[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) ev[j] = p0 + j < pr[i] ? glibc_expf(sv[j] - m[i]) : 0.0f;
-      const float4 e4 = make_float4(ev[0], ev[1], ev[2], ev[3]);
-      reinterpret_cast<float4*>(eb + (RPT * rg + i) * APT_ES)[pg] = e4;
-      if (pr[i] > p0) *scw(i, b) = e4;
-    }
-    __syncthreads();
-    if (tid < APT_R) {
-      const float* er = eb + tid * APT_ES;
-#pragma unroll 8
-      for (int p = 0; p < APT_PB; ++p) sum += er[p];
-    }
-    __syncthreads();
-  }
-  if (tid < APT_R) irow[tid] = 1.0f / sum;
-  APT_PUT()  // the first V block
-  __syncthreads();
-  float inv[RPT];
-#pragma unroll
-  for (int i = 0; i < RPT; ++i) inv[i] = irow[RPT * rg + i];
-  // ---- C: output sums
-  const int dgi = tid & 31;  // dims DB*dgi .. +DB-1 of rows RPT rg ..
-  float o[RPT][DB];
-#pragma unroll
-  for (int i = 0; i < RPT; ++i)
-#pragma unroll
-    for (int k = 0; k < DB; ++k) o[i][k] = 0.0f;
-#pragma unroll
-  for (int i = 0; i < RPT; ++i) snext[i] = pr[i] > 4 * pg ? *scw(i, 0) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  for (int b = 0; b < nblk; ++b) {
-    const int pb = b * APT_PB, p0 = pb + 4 * pg;
-    if (b + 1 < nblk) {
-      APT_LOAD_V(b + 1)
-    }
-    float4 ecur[RPT];
-#pragma unroll
-    for (int i = 0; i < RPT; ++i) ecur[i] = snext[i];
-    if (b + 1 < nblk) {
-#pragma unroll
-      for (int i = 0; i < RPT; ++i) snext[i] = pr[i] > p0 + APT_PB ? *scw(i, b + 1) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
-#pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-      const float ev[4] = {ecur[i].x, ecur[i].y, ecur[i].z, ecur[i].w};
-      float pv[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) pv[j] = p0 + j < pr[i] ? ev[j] * inv[i] : 0.0f;
-      reinterpret_cast<float4*>(eb + (RPT * rg + i) * APT_ES)[pg] = make_float4(pv[0], pv[1], pv[2], pv[3]);
-    }
-    __syncthreads();
-    const bool masked = pb + APT_PB > pmin;  // a row of the tile ends inside this block
-#pragma unroll 1
-    for (int gq = 0; gq < APT_PB / 8; ++gq) {
-      uint4 v[DB];
-#pragma unroll
-      for (int k = 0; k < DB; ++k) v[k] = kb[gq * HD + DB * dgi + k];
-      float pp[RPT][8];
-#pragma unroll
-      for (int i = 0; i < RPT; ++i) {
-        const float4 a = reinterpret_cast<const float4*>(eb + (RPT * rg + i) * APT_ES + 8 * gq)[0];
-        const float4 c = reinterpret_cast<const float4*>(eb + (RPT * rg + i) * APT_ES + 8 * gq)[1];
-        pp[i][0] = a.x; pp[i][1] = a.y; pp[i][2] = a.z; pp[i][3] = a.w;
-        pp[i][4] = c.x; pp[i][5] = c.y; pp[i][6] = c.z; pp[i][7] = c.w;
-      }
-      if (!masked) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-#pragma unroll
-          for (int i = 0; i < RPT; ++i)
-#pragma unroll
-            for (int k = 0; k < DB; ++k) o[i][k] += mul_gran(pp[i][e], v[k], e);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int p = pb + 8 * gq + e;
-#pragma unroll
-          for (int i = 0; i < RPT; ++i)
-#pragma unroll
-            for (int k = 0; k < DB; ++k) {
-              const float t = mul_gran(pp[i][e], v[k], e);
-              if (p < pr[i]) o[i][k] += t;
-            }
+        for (int i = 0; i < 4; ++i) {
+          s[i] = acc[4 * u + i] * scale;
+          if (p < pr[i]) rm[i] = fmaxf(rm[i], s[i]);
         }
+        *reinterpret_cast<float4*>(sc + ((size_t)lb * pitch + p) * 4) = make_float4(s[0], s[1], s[2], s[3]);
       }
     }
-    __syncthreads();  // every wave is done with this block's V and probabilities
-    if (b + 1 < nblk) {
-      APT_PUT()
-    }
-    // (the next block's probabilities are written after this barrier's successor)
-  }
-  __syncthreads();
-  // ---- outputs: rows to LDS (reusing the q tile), then one (row, 32-value block) per thread
-  float* os = qs;  // [64][HD]
+    // over the 16 lanes of a block
 #pragma unroll
-  for (int i = 0; i < RPT; ++i) {
-    const int r = RPT * rg + i;
+    for (int i = 0; i < 4; ++i) {
 #pragma unroll
-    for (int k = 0; k < DB; ++k) {
-      const int d = DB * dgi + k;
-      // a single position copies the V row (its bits, -0 included)
-      os[r * HD + d] = pr[i] == 1 ? half_bits_to_float(vc[hbase + kv_v_index(HD, 0, d)]) : o[i][k];
+      for (int o = 8; o >= 1; o >>= 1) rm[i] = fmaxf(rm[i], __shfl_xor(rm[i], o));
+      if (lr == 0) smax[wave][4 * lb + i] = rm[i];
     }
   }
   __syncthreads();
-  for (int i = tid; i < APT_R * (HD / 32); i += NT) {
-    const int r = i / (HD / 32), blk = i % (HD / 32);
-    if (prow[r] == 0) continue;
+
+  // ---- B: exponentials, each row's sum in position order
+  {
+    const int rq = RW / 4 * wave + lane % LP;  // this lane's row quad
+    float m[4];
+    int prb[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      m[i] = smax[0][4 * rq + i];
+#pragma unroll
+      for (int w = 1; w < W; ++w) m[i] = fmaxf(m[i], smax[w][4 * rq + i]);
+      prb[i] = row_p(4 * rq + i);
+    }
+    float* ew = eb[wave];
+    float sum = 0.0f;
+    const int pl = lane / LP;
+    const float* sp = sc + ((size_t)rq * pitch + pl) * 4;
+    // the transposed cells: lane = (cell of 4 positions, row) of the wave's rows
+    const int tr = lane % RW, tc = lane / RW;
+    float* tp = sc + ((size_t)(RW / 4 * wave + tr / 4) * pitch + 4 * tc) * 4 + 4 * (tr & 3);
+    float4 nx = *reinterpret_cast<const float4*>(sp);
+    for (int p0 = 0; p0 < pmax; p0 += PS) {
+      const float4 s4 = nx;
+      if (p0 + PS < pmax) nx = *reinterpret_cast<const float4*>(sp + (size_t)(p0 + PS) * 4);
+      const float s[4] = {s4.x, s4.y, s4.z, s4.w};
+      float e[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) e[i] = glibc_expf_nonpos_t(s[i] - m[i], etab);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        ew[(4 * (lane % LP) + i) * ES + pl] = p0 + pl < prb[i] ? e[i] : 0.0f;
+      // the LDS block is this wave's own: wave-level ordering only
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const float* er = ew + tr * ES;
+#pragma unroll
+      for (int k = 0; k < PS * RW / 256; ++k)  // (one cell per lane when RW = 4)
+        *reinterpret_cast<float4*>(tp + (size_t)(p0 + k * (256 / RW)) * 4) =
+            *reinterpret_cast<const float4*>(er + 4 * tc + k * (256 / RW));
+#pragma unroll
+      for (int k = 0; k < PS / 4; ++k) add4(sum, reinterpret_cast<const float4*>(er)[k]);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    if (lane < RW) sinv[RW * wave + lane] = 1.0f / sum;
+  }
+  __syncthreads();
+
+  // ---- C: output sums of dims 32 wave ..
+  {
+    const float inv = sinv[lr];
+    const int n16 = (pmax + 15) >> 4;  // steps of 16 positions
+    const int nfree = pmin >> 4;       // of them before any row's end
+    const int glast = (pmax - 1) >> 3;
+    const uint2* vp = vg + (32 * wave + 16 * (lb & 1) + lr) * 2 + (lb >> 1);
+    // exponentials of row lr: register c holds, in block b, position 16 s + 8 (b % 2) + 4 (b / 2) + c
+    const float* ep = sc + ((size_t)(lr >> 2) * pitch + 8 * (lb & 1) + 4 * (lb >> 1)) * 4 + 4 * (lr & 3);
+    float acc[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
+    constexpr int D = 3;  // steps in flight
+    uint2 vr[D][2];
+    float4 er[D];
+    auto load = [&](int k, int s) __attribute__((always_inline)) {
+      const int sl = min(s, n16 - 1);
+      vr[k][0] = vp[(size_t)(2 * sl) * HD * 2];
+      vr[k][1] = vp[(size_t)min(2 * sl + 1, glast) * HD * 2];
+      er[k] = *reinterpret_cast<const float4*>(ep + (size_t)sl * 64);
+    };
+    auto step = [&](int k, int s, auto mc) __attribute__((always_inline)) {
+      constexpr bool masked = decltype(mc)::value;
+      const float a[4] = {er[k].x * inv, er[k].y * inv, er[k].z * inv, er[k].w * inv};
+      int left[4], left8[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        left[i] = pr[i] - 16 * s;
+        left8[i] = left[i] - 8;
+      }
+      outer_terms<0, masked>(acc, a, vr[k][0], left);
+      outer_terms<1, masked>(acc, a, vr[k][1], left8);
+    };
+#pragma unroll
+    for (int k = 0; k < D; ++k) load(k, k);
+    int s = 0;
+    for (; s + D <= nfree; s += D) {
+#pragma unroll
+      for (int k = 0; k < D; ++k) {
+        step(k, s + k, gm_const<bool, false>{});
+        load(k, s + k + D);
+      }
+    }
+#pragma unroll 1
+    for (; s < n16; ++s) {  // the last steps: rows ending inside, or fewer than D left
+      step(0, s, gm_const<bool, true>{});
+#pragma unroll
+      for (int k = 0; k + 1 < D; ++k) {
+        vr[k][0] = vr[k + 1][0];
+        vr[k][1] = vr[k + 1][1];
+        er[k] = er[k + 1];
+      }
+      load(D - 1, s + D);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int d = 32 * wave + 16 * u + lr;
+        // a single position copies the V row (its bits, -0 included)
+        os[4 * lb + i][d] = pr[i] == 1 ? half_bits_to_float(vc[hbase + kv_v_index(HD, 0, d)]) : acc[4 * u + i];
+      }
+  }
+  __syncthreads();
+  // ---- outputs: one (row, 32-value block) per thread
+  if (tid < APM_R * (HD / 32)) {
+    const int r = tid / (HD / 32), blk = tid % (HD / 32);
+    if (r >= nr) return;
     float y[32];
 #pragma unroll
-    for (int e = 0; e < 32; ++e) y[e] = os[r * HD + 32 * blk + e];
-    const size_t o0 = (size_t)row_tok(r) * n_heads * HD + (size_t)row_head(r) * HD + 32 * blk;
+    for (int e = 0; e < 32; ++e) y[e] = os[r][32 * blk + e];
+    const size_t o0 = row_off(r) + 32 * blk;
     if (att_out) {
 #pragma unroll
       for (int e = 0; e < 32; e += 4)
@@ -890,9 +873,6 @@ __global__ __launch_bounds__(NT) void k_attn_prefill_tile(
     qp[0] = make_uint4(packed[0], packed[1], packed[2], packed[3]);
     qp[1] = make_uint4(packed[4], packed[5], packed[6], packed[7]);
   }
-#undef APT_LOAD_K
-#undef APT_LOAD_V
-#undef APT_PUT
 }
 
 // ---------------------------------------------------------------------------

@@ -514,6 +514,37 @@ def test_attention_prefill_bit_exact(native, orc, monkeypatch, nh, nkv, hd, pos0
         assert np.array_equal(_bits(gxs[t]), _bits(ws)) and np.array_equal(gxq[t], wq)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,pos0,T", [(5, 1, 128, 15, 7), (20, 1, 64, 31, 3), (3, 3, 64, 63, 18),
+                                             (6, 2, 128, 0, 16), (16, 8, 128, 112, 33), (8, 1, 64, 47, 2)])
+def test_attention_prefill_tile_edges(native, orc, monkeypatch, nh, nkv, hd, pos0, T):
+    """The tiled prefill attention where a tile's 16 rows cross tokens (heads per KV head that do
+    not divide 16, or more than 16), its last tile is partly empty, and rows end at, before and
+    after the 8-, 16-, 32- and 64-position boundaries of its phases.  The last token's K and V rows
+    hold infinities: they reach that token's rows alone.  Every value is the per-position
+    oracle's, bit for bit (an f32 sum in another order, or a masked term, would not be)."""
+    monkeypatch.setenv("CAMELID_HIP_ATT_TILE", "1")
+    rng = np.random.default_rng(nh * 7 + pos0 + T)
+    max_pos = (pos0 + T + 7) // 8 * 8
+    kf = rng.normal(0, 1.5, (1, nkv, max_pos, hd)).astype(np.float32)
+    vf = rng.normal(0, 1, (1, nkv, max_pos, hd)).astype(np.float32)
+    vf[:, :, pos0 + T - 1, ::3] = 1e6
+    kf[:, :, pos0 + T - 1, 5] = -1e6
+    kb, vb = orc.f32_to_f16(kf), orc.f32_to_f16(vf)
+    q = rng.normal(0, 1, (T, nh * hd)).astype(np.float32)
+    scale = float(np.float32(1) / np.sqrt(np.float32(hd)))
+    kd, vd = _kv_device(kb, vb)
+    dq, dk, dv = _dev(q), _dev(kd), _dev(vd)
+    out, xq, xs = _buf(T * nh * hd * 4), _buf(T * nh * hd), _buf(T * nh * hd // 32 * 4)
+    _ok(native.camelid_hip_attention_prefill(dq.ptr, dk.ptr, dv.ptr, 0, nh, nkv, hd, max_pos, pos0, T, scale,
+                                             out.ptr, xq.ptr, xs.ptr, None))
+    got = out.download(np.float32, T * nh * hd).reshape(T, nh * hd)
+    kl, vl = orc.f16_to_f32(kb[0]).ravel(), orc.f16_to_f32(vb[0]).ravel()
+    for t in range(T):
+        want = orc.attention(q[t], kl, vl, nh, nkv, hd, max_pos, pos0 + t + 1)
+        same = (_bits(got[t]) == _bits(want)) | (np.isnan(got[t]) & np.isnan(want))
+        assert same.all(), f"token {t}"
+
+
 def test_quantize_q8_k_bit_exact(native, orc):
     """Q8_K activation quantizer == quantize_q8_k_blocks, incl. zero blocks, |max| ties (first
     wins), one-hot and huge/tiny blocks; per-32 sums of the quants."""
