@@ -44,17 +44,7 @@ struct Q8Mat {
   int8_t* q = nullptr;
   uint16_t* d = nullptr;
   uint32_t rows = 0, k = 0;
-  // a weight scale is +-inf (or not known not to be): the prefill GEMM folds with the plain
-  // conversion and product (cm::k_gemm_q8<true, NF>), which gives dot * inf; else with one FMA
-  bool inf_scale = true;
 };
-
-// Whether any of the n f16 values is +-inf.
-bool f16_any_inf(const uint16_t* h, size_t n) {
-  for (size_t i = 0; i < n; ++i)
-    if ((h[i] & 0x7fffu) == 0x7c00u) return true;
-  return false;
-}
 
 // A K-quant matrix as planes split out of its GGUF superblocks (kernels_kquant.h):
 // Q4_K: a = nibbles [rows][k/2], b = headers [rows][k/256][16];
@@ -345,7 +335,6 @@ int upload_q8(camelid_hip_engine* e, Q8Mat* m, const std::vector<Part>& parts, u
   }
   m->rows = rows;
   m->k = k;
-  m->inf_scale = f16_any_inf(d.data(), d.size());
   HIP_TRY(e, hipMemcpy(m->q, q.data(), q.size(), hipMemcpyHostToDevice));
   HIP_TRY(e, hipMemcpy(m->d, d.data(), d.size() * 2, hipMemcpyHostToDevice));
   return 0;
@@ -1449,7 +1438,10 @@ void launch_kgemm(const KMat& m, uint32_t T, const float* kd, const int8_t* kq, 
   }
 }
 
-constexpr int GEMM_NF1_BELOW = 512;
+// 64 x 64 tiles from this many of them on (256 CUs), else 32 x 32 ones.  Measured (us, 64 / 32):
+// [3072 x 3072] 200 tokens (192 tiles of 64) 26.3 / 20.1, 300 (240) 26.2 / 24.6, 511 (384) 31.5 /
+// 34.3; [11264 x 2048] 37 tokens (176) 18.2 / 13.9, 127 (352) 22.7 / 24.7.
+constexpr int GEMM_BIG_TILES = 288;
 void launch_gemm(const Q8Mat& m, uint32_t T, const int8_t* xq, const float* xs, float* y, const float* resid,
                  hipStream_t s) {
   if (T <= (uint32_t)cm::GMT_MAX && m.k <= 8192) {  // a few tokens: weights streamed once by GEMV-shaped workgroups
@@ -1466,44 +1458,18 @@ void launch_gemm(const Q8Mat& m, uint32_t T, const int8_t* xq, const float* xs, 
         break;
     }
   }
-  // 32-row tiles when 64-row ones give fewer than two workgroups per CU of the 256 (measured
-  // at 512 tokens: [2048 x 2048] 20.5 -> 18.1 us, [2048 x 5632] 52.8 -> 46.2 us with them; at
-  // 704 tiles, [5632 x 2048], 36.3 -> 40.4 us, so not there).  CAMELID_HIP_GEMM_NF=1 / 2
-  // forces either tile height.
-  int nf = cm::gemm_tiles((int)m.rows, (int)T, 2) < GEMM_NF1_BELOW ? 1 : 2;
+  // CAMELID_HIP_GEMM_NF=1 / 2 forces the 32 / 64 tiles
+  bool big = cm::gm_tiles((int)m.rows, (int)T, 32) >= GEMM_BIG_TILES;
   if (const char* f = std::getenv("CAMELID_HIP_GEMM_NF")) {
-    if (f[0] == '1') nf = 1;
-    if (f[0] == '2') nf = 2;
+    if (f[0] == '1') big = false;
+    if (f[0] == '2') big = true;
   }
-#define CM_GEMM(PLAIN, NF)                                                                                      \
-  CM_LAUNCH((cm::k_gemm_q8<PLAIN, NF>), dim3(cm::gemm_grid((int)m.rows, (int)T, NF)), dim3(cm::GM_NT), 0, s, m.q, \
-            m.d, (int)m.rows, (int)m.k, xq, xs, (int)T, y, resid)
-  if (m.inf_scale) {
-    if (nf == 1) CM_GEMM(true, 1);
-    else CM_GEMM(true, 2);
-  } else {
-    if (nf == 1) CM_GEMM(false, 1);
-    else CM_GEMM(false, 2);
-  }
-#undef CM_GEMM
-}
-
-// Q8Mat::inf_scale of weight scales already on the device (the entry points that take device
-// pointers): a scan on the stream, its flag read back (synchronizes the stream).
-int q8_scan_inf_scales(Q8Mat* m, hipStream_t s) {
-  const size_t n = (size_t)m->rows * (m->k / 32);
-  uint32_t* flag = nullptr;
-  uint32_t h = 1;
-  if (hipMalloc(&flag, 4) != hipSuccess) return fail(nullptr, "scale scan: device allocation failed");
-  const uint32_t grid = (uint32_t)std::min<size_t>((n + 255) / 256, 1024);
-  bool ok = hipMemsetAsync(flag, 0, 4, s) == hipSuccess;
-  if (ok) hipLaunchKernelGGL(cm::k_f16_any_inf, dim3(grid), dim3(256), 0, s, m->d, n, flag);
-  ok = ok && hipGetLastError() == hipSuccess && hipMemcpyAsync(&h, flag, 4, hipMemcpyDeviceToHost, s) == hipSuccess &&
-       hipStreamSynchronize(s) == hipSuccess;
-  (void)hipFree(flag);
-  if (!ok) return fail(nullptr, "scale scan failed");
-  m->inf_scale = h != 0;
-  return 0;
+  if (big)
+    CM_LAUNCH((cm::k_gemm_q8<32, 4, false>), dim3(cm::gm_grid((int)m.rows, (int)T, 32)), dim3(cm::GM_NT), 0, s, m.q,
+              m.d, (int)m.rows, (int)m.k, xq, xs, (int)T, y, resid);
+  else
+    CM_LAUNCH((cm::k_gemm_q8<16, 8, true>), dim3(cm::gm_grid((int)m.rows, (int)T, 16)), dim3(cm::GM_NT), 0, s, m.q,
+              m.d, (int)m.rows, (int)m.k, xq, xs, (int)T, y, resid);
 }
 
 // Whether the tiled attention of a prefill chunk (cm::k_attn_prefill_mm: 16 rows of a KV head per
@@ -2762,7 +2728,6 @@ int camelid_hip_q8_0_gemm(const int8_t* wq, const uint16_t* wd, uint32_t rows, u
   m.d = const_cast<uint16_t*>(wd);
   m.rows = rows;
   m.k = k;
-  if (q8_scan_inf_scales(&m, (hipStream_t)stream)) return 1;
   launch_gemm(m, tokens, xq, xs, y, resid, (hipStream_t)stream);
   return launch_status("q8_0_gemm");
 }
@@ -2890,12 +2855,11 @@ int camelid_hip_time_q8_0(int batched, const int8_t* const* wq, const uint16_t* 
     rc = fail(nullptr, "event create failed");
   } else {
     std::vector<Q8Mat> mats(copies);
-    for (uint32_t c = 0; c < copies && !rc; ++c) {
+    for (uint32_t c = 0; c < copies; ++c) {
       mats[c].q = const_cast<int8_t*>(wq[c]);
       mats[c].d = const_cast<uint16_t*>(wd[c]);
       mats[c].rows = rows;
       mats[c].k = k;
-      if (batched) rc = q8_scan_inf_scales(&mats[c], s);
     }
     auto launch = [&](uint32_t i) {
       const Q8Mat& m = mats[i % copies];

@@ -11,282 +11,11 @@
 //   SwiGLU           k_silu_rows
 #pragma once
 #include "kernels_decode.h"
+#include "kernels_gemm_q8.h"
 
 namespace cm {
 
 typedef int v4i_t __attribute__((ext_vector_type(4)));
-
-// ---------------------------------------------------------------------------
-// Q8_0 GEMM (q8_gemm_batched, cuda_resident.rs:1494; CPU: the row dot of
-// inference.rs:19871-19905 per token):
-//   y[t][n] = (resid ? resid[t][n] : 0) + fold_b (float(dot_b(W[n], X[t])) * wd[n][b]) * xs[t][b]
-// with dot_b the exact int32 dot of one 32-value block and the fold in block order from 0.
-// The block dots run on the matrix cores: one v_mfma_i32_16x16x32_i8 per 16x16 (rows x
-// tokens) fragment and block; its K = 32 is exactly one Q8_0 block, so every block's int32
-// dot comes out separately (any assignment of the 32 byte positions to lanes gives the same
-// integer, as long as the weight and activation operands use the same one).
-// Workgroup: 4 waves over a (32 NF)-row x 64-token tile, each wave 16 NF x 32 (NF x 2 fragments).
-// Lane l of a fragment supplies row / token l % 16, bytes 8*(l/16) .. +7 of the block, and
-// receives the outputs of rows 4*(l/16) + i (i = 0..3) for token l % 16.
-// Operands move in steps of 4 blocks (128 bytes of every row and token): coalesced 16-byte
-// global loads into registers one step ahead, then into a double-buffered LDS tile laid out
-// [block][8-byte piece][row] (a fragment read is 16 consecutive 8-byte pieces per piece
-// index: no bank conflicts).  Scales are staged in LDS 8 blocks at a time (transposed:
-// [block][row], [block][token]), the next group's held in registers meanwhile.
-// Tiles are dealt so that each XCD (workgroup id mod 8) runs a contiguous range of tiles,
-// token tiles innermost: the row tile's weights are read once per XCD and re-read from its L2.
-// N % 4 == 0 (16-byte output stores); K % 32 == 0; y may alias resid.
-constexpr int GM_NT = 256;
-constexpr int GM_RT = 64;  // tokens per workgroup tile
-constexpr int GM_BG = 8;   // blocks per scale-staging group
-constexpr int GM_SB = 4;   // blocks per operand step
-// Rows per workgroup tile: 32 * NF, NF = 2 (64) or 1 (32, for small grids: a [3072 x 3072] x 511
-// product has 384 tiles of 64 x 64, one or two 4-wave workgroups per CU, and a single wave
-// issues one VALU instruction per ~7 clocks, so each SIMD then idles half the time).
-__host__ __device__ constexpr int gm_rows(int NF) { return 32 * NF; }
-// 8-byte pieces per [block][piece] row of an LDS operand tile: rows + 1 pad, so that the
-// planes start 2 banks apart (2 * rows + 2 dwords) and the 8 pieces a row's 16-byte chunks
-// scatter to land in different banks (the tile writes are otherwise 8-way bank conflicts)
-__host__ __device__ constexpr int gm_ps(int rows) { return rows + 1; }
-// The block dots start from the bit pattern of 1.5 * 2^23 instead of 0: |dot| <= 32 * 128^2
-// = 2^19 < 2^22, so the int32 sum's bits are those of the f32 value 1.5 * 2^23 + dot (ulp 1
-// in [2^23, 2^24)), and fma(f, w, -(1.5 * 2^23) w) = round(f w - 1.5 * 2^23 w) = round(dot w)
-// exactly (the FMA rounds once, -(1.5 * 2^23) w is exact for every f16 w: 13 significant
-// bits, no overflow).  That is float(dot) * w in one mixed-precision FMA, in place of a
-// conversion and a multiply.  An infinite w (dot * w = +-inf, or NaN at dot = 0) is the one
-// value it does not give: a matrix whose weight scales hold one runs k_gemm_q8<true, NF>, the
-// plain form (the host decides per matrix).
-constexpr int32_t GM_MAGIC = 0x4B400000;
-constexpr float GM_MAGIC_F = 12582912.0f;
-
-// a * f32(lo / hi half of w) + c, rounded once: one v_fma_mix_f32.  Written as an fma of the
-// widened half (not inline assembly): the operand a comes straight from a matrix-core result,
-// and only compiler-visible reads get the wait states the hardware needs after an MFMA write.
-__device__ __forceinline__ float fma_f16_lo(float a, uint32_t w, float c) {
-  _Float16 h[2];
-  __builtin_memcpy(h, &w, 4);
-  return __builtin_fmaf(a, (float)h[0], c);
-}
-__device__ __forceinline__ float fma_f16_hi(float a, uint32_t w, float c) {
-  _Float16 h[2];
-  __builtin_memcpy(h, &w, 4);
-  return __builtin_fmaf(a, (float)h[1], c);
-}
-
-template <typename V, V X>
-struct gm_const {
-  static constexpr V value = X;
-};
-
-__host__ __device__ inline int gemm_tiles(int N, int T, int NF = 2) {
-  return ((N + gm_rows(NF) - 1) / gm_rows(NF)) * ((T + GM_RT - 1) / GM_RT);
-}
-__host__ __device__ inline int gemm_grid(int N, int T, int NF = 2) { return ((gemm_tiles(N, T, NF) + 7) / 8) * 8; }
-
-// PLAIN: the dots from 0, converted and multiplied by the weight scale (two VALU operations);
-// else from the 1.5 * 2^23 pattern, one FMA (GM_MAGIC).  Both give float(dot) * w rounded
-// once, then * xs, then + in block order.
-// Waves: 2 (rows) x 2 (tokens), each 16 NF rows x 32 tokens (NF x 2 fragments).
-// (at most 128 VGPRs and, with 8-block scale groups, under 40 KB of LDS: four workgroups per CU)
-template <bool PLAIN, int NF>
-__global__ __launch_bounds__(GM_NT, 4) void k_gemm_q8(const int8_t* __restrict__ wq, const uint16_t* __restrict__ wd,
-                                                   int N, int K, const int8_t* __restrict__ xq,
-                                                   const float* __restrict__ xs, int T, float* y,
-                                                   const float* resid) {
-  constexpr int RN = gm_rows(NF), PSA = gm_ps(RN), PSB = gm_ps(GM_RT);
-  constexpr int AJ = RN / 32, BJ = GM_RT / 32;  // 16-byte global loads per thread and step
-  static_assert((NF == 1 || NF == 2) && GM_RT == 64 && GM_NT == 256 && GM_SB == 4 && GM_BG % GM_SB == 0 &&
-                    GM_NT % GM_BG == 0, "tile layout");
-  __shared__ __align__(16) uint2 sa[2][GM_SB][4][PSA];
-  __shared__ __align__(16) uint2 sb[2][GM_SB][4][PSB];
-  __shared__ __align__(16) uint16_t swd[GM_BG][RN + 4];
-  __shared__ __align__(16) float snb[GM_BG][RN + 4];  // -(1.5 * 2^23) * f32(wd)
-  __shared__ __align__(16) float sxs[GM_BG][GM_RT + 1];
-  const int NB = K >> 5;
-  const int nsteps = (NB + GM_SB - 1) / GM_SB;
-  const int ntt = (T + GM_RT - 1) / GM_RT;
-  const int tiles = gemm_tiles(N, T, NF);
-  const int per = (tiles + 7) >> 3;
-  const int L = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-  if (L >= tiles) return;
-  const int n_base = (L / ntt) * RN, t_base = (L % ntt) * GM_RT;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int r = lane & 15, g = lane >> 4;
-  const int wn = (wave & 1) * 16 * NF, wt = (wave >> 1) * 32;
-
-  // global -> register loads of one step: chunk j of thread tid is 16 bytes of row / token
-  // (tid + 256 j) / 8 at byte (tid % 8) * 16 of the step's 128
-  const int crow = tid >> 3, cc = tid & 7;
-  const int8_t* ga[AJ];
-  const int8_t* gb[BJ];
-#pragma unroll
-  for (int j = 0; j < AJ; ++j) ga[j] = wq + (size_t)min(n_base + crow + 32 * j, N - 1) * K;
-#pragma unroll
-  for (int j = 0; j < BJ; ++j) gb[j] = xq + (size_t)min(t_base + crow + 32 * j, T - 1) * K;
-  uint4 ra[AJ], rb[BJ];
-  auto gload = [&](int step) __attribute__((always_inline)) {
-    const int off = min(step * 128 + cc * 16, K - 16);
-#pragma unroll
-    for (int j = 0; j < AJ; ++j) ra[j] = *reinterpret_cast<const uint4*>(ga[j] + off);
-#pragma unroll
-    for (int j = 0; j < BJ; ++j) rb[j] = *reinterpret_cast<const uint4*>(gb[j] + off);
-  };
-  auto lds_put = [&](int buf) __attribute__((always_inline)) {  // bytes 0..7 -> piece 2(cc%2), 8..15 -> piece 2(cc%2)+1
-    const int bl = cc >> 1, pc = (cc & 1) * 2;
-#pragma unroll
-    for (int j = 0; j < AJ; ++j) {
-      sa[buf][bl][pc][crow + 32 * j] = make_uint2(ra[j].x, ra[j].y);
-      sa[buf][bl][pc + 1][crow + 32 * j] = make_uint2(ra[j].z, ra[j].w);
-    }
-#pragma unroll
-    for (int j = 0; j < BJ; ++j) {
-      sb[buf][bl][pc][crow + 32 * j] = make_uint2(rb[j].x, rb[j].y);
-      sb[buf][bl][pc + 1][crow + 32 * j] = make_uint2(rb[j].z, rb[j].w);
-    }
-  };
-
-  // scale staging: thread tid carries block tid % GM_BG of rows / tokens tid / GM_BG + 16 i
-  constexpr int SPW = GM_BG * RN / GM_NT, SPX = GM_BG * GM_RT / GM_NT, SRS = GM_NT / GM_BG;
-  uint32_t pw[SPW];
-  float px[SPX];
-  auto stage_load = [&](int g0) __attribute__((always_inline)) {
-    const int blk = min(g0 + (tid % GM_BG), NB - 1);
-#pragma unroll
-    for (int i = 0; i < SPW; ++i) pw[i] = wd[(size_t)min(n_base + tid / GM_BG + SRS * i, N - 1) * NB + blk];
-#pragma unroll
-    for (int i = 0; i < SPX; ++i) px[i] = xs[(size_t)min(t_base + tid / GM_BG + SRS * i, T - 1) * NB + blk];
-  };
-  auto stage_store = [&]() __attribute__((always_inline)) {
-    const int bb = tid % GM_BG;
-#pragma unroll
-    for (int i = 0; i < SPW; ++i) {
-      const int row = tid / GM_BG + SRS * i;
-      swd[bb][row] = (uint16_t)pw[i];
-      if (!PLAIN) snb[bb][row] = -GM_MAGIC_F * half_bits_to_float((uint16_t)pw[i]);
-    }
-#pragma unroll
-    for (int i = 0; i < SPX; ++i) sxs[bb][tid / GM_BG + SRS * i] = px[i];
-  };
-
-  float acc[NF][2][4];
-#pragma unroll
-  for (int nf = 0; nf < NF; ++nf)
-#pragma unroll
-    for (int tf = 0; tf < 2; ++tf)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[nf][tf][i] = 0.0f;
-
-  // block b = step block bl, from LDS buffer buf
-  auto block = [&](int buf, int bl, int b) __attribute__((always_inline)) {
-    constexpr bool plain = PLAIN;
-    long av[NF], bv[2];
-#pragma unroll
-    for (int f = 0; f < NF; ++f) av[f] = *reinterpret_cast<const long*>(&sa[buf][bl][g][wn + 16 * f + r]);
-#pragma unroll
-    for (int f = 0; f < 2; ++f) bv[f] = *reinterpret_cast<const long*>(&sb[buf][bl][g][wt + 16 * f + r]);
-    const int32_t c0 = plain ? 0 : GM_MAGIC;
-    v4i_t c[NF][2];
-#pragma unroll
-    for (int nf = 0; nf < NF; ++nf)
-#pragma unroll
-      for (int tf = 0; tf < 2; ++tf)
-        c[nf][tf] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[nf], bv[tf], v4i_t{c0, c0, c0, c0}, 0, 0, 0);
-    const int sl = b & (GM_BG - 1);
-    uint2 w2[NF];
-    float4 nb[NF];
-    float xv[2];
-#pragma unroll
-    for (int nf = 0; nf < NF; ++nf) {
-      w2[nf] = *reinterpret_cast<const uint2*>(&swd[sl][wn + 16 * nf + 4 * g]);
-      if (!plain) nb[nf] = *reinterpret_cast<const float4*>(&snb[sl][wn + 16 * nf + 4 * g]);
-    }
-#pragma unroll
-    for (int tf = 0; tf < 2; ++tf) xv[tf] = sxs[sl][wt + 16 * tf + r];
-#pragma unroll
-    for (int nf = 0; nf < NF; ++nf)
-#pragma unroll
-      for (int tf = 0; tf < 2; ++tf) {
-        if (plain) {
-          acc[nf][tf][0] += mul_f16_lo((float)c[nf][tf][0], w2[nf].x) * xv[tf];
-          acc[nf][tf][1] += mul_f16_hi((float)c[nf][tf][1], w2[nf].x) * xv[tf];
-          acc[nf][tf][2] += mul_f16_lo((float)c[nf][tf][2], w2[nf].y) * xv[tf];
-          acc[nf][tf][3] += mul_f16_hi((float)c[nf][tf][3], w2[nf].y) * xv[tf];
-        } else {
-          acc[nf][tf][0] += fma_f16_lo(__int_as_float(c[nf][tf][0]), w2[nf].x, nb[nf].x) * xv[tf];
-          acc[nf][tf][1] += fma_f16_hi(__int_as_float(c[nf][tf][1]), w2[nf].x, nb[nf].y) * xv[tf];
-          acc[nf][tf][2] += fma_f16_lo(__int_as_float(c[nf][tf][2]), w2[nf].y, nb[nf].z) * xv[tf];
-          acc[nf][tf][3] += fma_f16_hi(__int_as_float(c[nf][tf][3]), w2[nf].y, nb[nf].w) * xv[tf];
-        }
-      }
-    // the folds stay in this block (not sunk past the staging branch with the dots held live)
-#pragma unroll
-    for (int nf = 0; nf < NF; ++nf)
-#pragma unroll
-      for (int tf = 0; tf < 2; ++tf)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(acc[nf][tf][i]));
-  };
-  // operand step s from LDS buffer s % 2, GM_SB blocks (FULL) or the NB % GM_SB of the last
-  // step; then the next step's operands into the other buffer
-  auto run_step = [&](int s, auto fullc) __attribute__((always_inline)) {
-    constexpr bool full = decltype(fullc)::value;
-    const int buf = s & 1, b0 = s * GM_SB;
-    if (s + 1 < nsteps) gload(s + 1);
-    if (full) {
-      block(buf, 0, b0);
-      block(buf, 1, b0 + 1);
-      block(buf, 2, b0 + 2);
-      block(buf, 3, b0 + 3);
-    } else {
-      for (int bl = 0; bl < NB - b0; ++bl) block(buf, bl, b0 + bl);
-    }
-    if (s + 1 < nsteps && ((s + 1) * GM_SB) % GM_BG == 0) {  // next step opens a new scale group
-      lds_put(buf ^ 1);
-      __syncthreads();  // every wave is done with this group's scales
-      stage_store();
-      const int g_next = (s + 1) * GM_SB + GM_BG;
-      if (g_next < NB) stage_load(g_next);
-      __syncthreads();
-    } else {
-      if (s + 1 < nsteps) lds_put(buf ^ 1);
-      __syncthreads();
-    }
-  };
-
-  stage_load(0);
-  gload(0);
-  stage_store();
-  if (GM_BG < NB) stage_load(GM_BG);
-  lds_put(0);
-  __syncthreads();
-  const int nfull = NB / GM_SB;
-  for (int s = 0; s < nfull; ++s) run_step(s, gm_const<bool, true>{});
-  if (nfull < nsteps) run_step(nfull, gm_const<bool, false>{});  // the partial last step
-#pragma unroll
-  for (int nf = 0; nf < NF; ++nf)
-#pragma unroll
-    for (int tf = 0; tf < 2; ++tf) {
-      const int t = t_base + wt + 16 * tf + r, n = n_base + wn + 16 * nf + 4 * g;
-      if (t < T && n < N) {
-        const size_t o = (size_t)t * N + n;
-        float4 v = make_float4(acc[nf][tf][0], acc[nf][tf][1], acc[nf][tf][2], acc[nf][tf][3]);
-        if (resid) {
-          const float4 rr = *reinterpret_cast<const float4*>(resid + o);
-          v = make_float4(rr.x + v.x, rr.y + v.y, rr.z + v.z, rr.w + v.w);
-        }
-        *reinterpret_cast<float4*>(y + o) = v;
-      }
-    }
-}
-
-// Sets *flag (cleared by the caller) when one of the n f16 values is +-inf: which fold form a
-// matrix of device-resident weight scales needs (k_gemm_q8<true> if set).
-__global__ __launch_bounds__(256) void k_f16_any_inf(const uint16_t* __restrict__ h, size_t n, uint32_t* flag) {
-  bool inf = false;
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
-    inf |= (h[i] & 0x7fffu) == 0x7c00u;
-  if (inf) *flag = 1u;  // every writer stores the same value
-}
 
 // ---------------------------------------------------------------------------
 // Greedy argmax (inference.rs:5912-5925: first index of the max, strict '>') of T rows of n
@@ -829,13 +558,13 @@ __global__ __launch_bounds__(HD * 2, 4) void k_attn_prefill_mm(
     for (; s + D <= nfree; s += D) {
 #pragma unroll
       for (int k = 0; k < D; ++k) {
-        step(k, s + k, gm_const<bool, false>{});
+        step(k, s + k, std::false_type{});
         load(k, s + k + D);
       }
     }
 #pragma unroll 1
     for (; s < n16; ++s) {  // the last steps: rows ending inside, or fewer than D left
-      step(0, s, gm_const<bool, true>{});
+      step(0, s, std::true_type{});
 #pragma unroll
       for (int k = 0; k + 1 < D; ++k) {
         vr[k][0] = vr[k + 1][0];

@@ -131,6 +131,23 @@ def test_q8_gemm_forced_tile_height(native, orc, monkeypatch, rows, k, tokens, n
     assert np.array_equal(_bits(dres.download(np.float32, tokens * rows).reshape(tokens, rows)), _bits(resid + want))
 
 
+@pytest.mark.parametrize("nf", ["1", "2"])
+@pytest.mark.parametrize("rows,k,tokens", [(4, 32, 9), (68, 96, 31), (32, 288, 33), (100, 544, 64), (64, 1056, 17)])
+def test_q8_gemm_step_edges(native, orc, monkeypatch, rows, k, tokens, nf):
+    """Both tilings where the blocks of a row do not fill a staging step (1, 3, 9, 17 and 33 of
+    them, steps of 4 and 8), and rows and tokens one short of, at and past a 32 or 64 tile."""
+    monkeypatch.setenv("CAMELID_HIP_GEMM_NF", nf)
+    rng = np.random.default_rng(rows + 3 * k + tokens)
+    wire = orc.quantize_q8_0_wire(rng.normal(0, 0.02, rows * k).astype(np.float32))
+    q, d = _repack(native, wire, rows, k)
+    pairs = [orc.quantize_q8_0(rng.normal(0, 1 + t % 5, k).astype(np.float32)) for t in range(tokens)]
+    xs, xq = np.stack([p[0] for p in pairs]), np.stack([p[1] for p in pairs])
+    wq, wd, dxq, dxs, y = _dev(q), _dev(d), _dev(xq), _dev(xs), _buf(rows * tokens * 4)
+    _ok(native.camelid_hip_q8_0_gemm(wq.ptr, wd.ptr, rows, k, dxq.ptr, dxs.ptr, tokens, y.ptr, None, None))
+    want = np.stack([orc.q8_0_gemv(wire, rows, k, xs[t], xq[t]) for t in range(tokens)])
+    assert np.array_equal(_bits(y.download(np.float32, rows * tokens).reshape(tokens, rows)), _bits(want))
+
+
 @pytest.mark.parametrize("rows,k", [(32000, 2048), (128256, 3072)])
 def test_q8_gemm_bit_exact_large(native, orc, rows, k):
     """The sweep's two largest shapes (TinyLlama's and Llama-3.2-3B's lm_head widths) at the
