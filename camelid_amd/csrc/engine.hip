@@ -1444,7 +1444,7 @@ void launch_kgemm(const KMat& m, uint32_t T, const float* kd, const int8_t* kq, 
 constexpr int GEMM_BIG_TILES = 288;
 void launch_gemm(const Q8Mat& m, uint32_t T, const int8_t* xq, const float* xs, float* y, const float* resid,
                  hipStream_t s) {
-  if (T <= (uint32_t)cm::GMT_MAX && m.k <= 8192) {  // a few tokens: weights streamed once by GEMV-shaped workgroups
+  if (T <= (uint32_t)cm::GMT_MAX && m.k <= 8192) {  // one or two tokens
     const uint32_t grid = (m.rows + cm::GMT_ROWS - 1) / cm::GMT_ROWS;
     const size_t lds = cm::gemv_multi_lds_bytes((int)m.k, (int)T);
     switch (m.k) {
@@ -1457,6 +1457,14 @@ void launch_gemm(const Q8Mat& m, uint32_t T, const int8_t* xq, const float* xs, 
       default:
         break;
     }
+  }
+  // a few tokens: weights streamed once by GEMV-shaped workgroups (16-byte loads of the scales too)
+  if (T <= (uint32_t)cm::GMM_MAX && m.k % cm::GMM_SEG == 0 &&
+      ((reinterpret_cast<uintptr_t>(m.d) | reinterpret_cast<uintptr_t>(xs)) & 15) == 0) {
+    CM_LAUNCH(cm::k_gemv_mm, dim3(cm::gemv_mm_grid((int)m.rows, (int)m.k)),
+              dim3(64 * cm::gemv_mm_waves((int)m.k)), cm::gemv_mm_lds_bytes((int)m.k), s, m.q, m.d, (int)m.rows,
+              (int)m.k, xq, xs, (int)T, y, resid);
+    return;
   }
   // CAMELID_HIP_GEMM_NF=1 / 2 forces the 32 / 64 tiles
   bool big = cm::gm_tiles((int)m.rows, (int)T, 32) >= GEMM_BIG_TILES;

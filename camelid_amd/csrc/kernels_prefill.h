@@ -65,13 +65,13 @@ __global__ __launch_bounds__(64) void k_argmax_rows_finish(const float* __restri
 }
 
 // ---------------------------------------------------------------------------
-// Y[t] = W . X[t] (+ resid[t]) for 1 <= T <= GMT_MAX tokens (speculative verify, short
-// prefill chunks): the single-token GEMV's arithmetic for every (row, token) -- exact int32
+// Y[t] = W . X[t] (+ resid[t]) for 1 <= T <= GMT_MAX tokens (the shortest verify and
+// prefill chunks; k_gemv_mm from four on): the single-token GEMV's arithmetic for every (row, token) -- exact int32
 // block dots, terms ((float)dot * d_w) * d_x, the in-order fold over blocks -- with each
 // weight chunk loaded once and dotted with all T activations (a 64-token matrix-core tile
 // would leave most CUs idle at this size).  4 waves x GMT_RPW rows per workgroup.
 // Dynamic LDS: gemv_multi_lds_bytes(K, T).
-constexpr int GMT_MAX = 8;
+constexpr int GMT_MAX = 3;
 constexpr int GMT_RPW = 1;
 constexpr int GMT_ROWS = 4 * GMT_RPW;
 // LDS: the activations [T][K] i8 and their scales [T][K/32] f32, each rounded up to whole
@@ -170,6 +170,181 @@ __global__ __launch_bounds__(256) void k_gemv_multi(const int8_t* __restrict__ w
       const size_t o = (size_t)tk * rows + row;
       y[o] = resid ? resid[o] + acc : acc;
     }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The same on the matrix cores for 1 <= T <= GMM_MAX tokens (speculative verify, short
+// prefill chunks): the single-token GEMV's arithmetic for every (row, token) -- exact int32
+// block dots, terms ((float)dot * d_w) * d_x, the in-order fold over blocks.
+// One v_mfma_i32_16x16x64_i8 gives the dots of 16 rows with 8 tokens for TWO blocks: the weights
+// are the B operand as they lie in memory (lane (n, g): bytes 16 g .. +15 of 64 of row n), the
+// activations the A operand, its 16 rows being (token, block of the two), zero in the other
+// block's half of K.  Row m is token 2 (m / 4) + m % 2 and block m / 2 % 2, so lane (n, g) gets
+// tokens 2 g, 2 g + 1 of row n in both blocks, and every lane's four terms are wanted.
+// Workgroup: 16 rows; each wave takes GMM_SEG values of K, all its loads in flight at once (8 KB
+// of weights per wave, plain loads: a 128-byte line is the two halves of two loads, and streaming
+// ones fetched it twice: the large shape below 106 us), and leaves its terms in LDS; then one wave
+// per token of the pair adds them in block order, reading a segment ahead.  The grid is what the
+// device holds: a wave's activations stay in its registers over all its row tiles, and the next
+// tile's weights are on their way while this one's terms are formed and added.  More than
+// GMM_WAVES segments go in slices with the sums carried along.
+// Bound by HBM on large matrices, by the latency of one load, product and fold on small ones.
+// Measured, 8 tokens (us, k_gemv_multi / this): [16384 x 3072] 26.1 / 14.9, [5120 x 3072]
+// 10.1 / 8.6, [3072 x 3072] 7.8 / 5.9, [3072 x 8192] 24.9 / 11.4, [128256 x 3072] 165 / 82 (5.1
+// TB/s), [28672 x 4096] 58.8 / 31.8; 4 tokens: [16384 x 3072] 15.0 / 14.3, [3072 x 3072] 6.1 / 5.8;
+// 3 tokens: 13.6 / 14.3, [5120 x 3072] 7.0 / 8.2, [28672 x 4096] 25.6 / 30.7, [128256 x 3072] 77.6 / 77.8.
+// K % GMM_SEG == 0; scales of either side 16-byte aligned.
+constexpr int GMM_MAX = 8;
+constexpr int GMM_SEG = 512;   // values of K per wave and slice: 8 chunks of two blocks
+constexpr int GMM_WAVES = 16;  // waves of a workgroup at most
+constexpr int GMM_ROWS = 16;
+// waves per workgroup (the last one idle in the products at K = 512: the fold wants two)
+inline int gemv_mm_waves(int K) {
+  const int segs = K / GMM_SEG, slices = (segs + GMM_WAVES - 1) / GMM_WAVES;
+  const int w = (segs + slices - 1) / slices;
+  return w < 2 ? 2 : w;
+}
+// per wave: the terms of a segment, then its activation scales [two chunks][token][block]
+constexpr int GMM_WAVE_LDS = 8 * 64 * 16 + GMM_MAX * (GMM_SEG / 32) * 4;
+inline size_t gemv_mm_lds_bytes(int K) { return (size_t)gemv_mm_waves(K) * GMM_WAVE_LDS; }
+// resident workgroups (four waves per SIMD at 128 registers; their LDS fits too)
+inline int gemv_mm_grid(int rows, int K) {
+  const int tiles = (rows + GMM_ROWS - 1) / GMM_ROWS, res = 256 * (16 / gemv_mm_waves(K));
+  return tiles < res ? tiles : res;
+}
+
+__global__ __launch_bounds__(GMM_WAVES * 64) void k_gemv_mm(const int8_t* __restrict__ wq,
+                                                               const uint16_t* __restrict__ wd, int rows, int K,
+                                                               const int8_t* __restrict__ xq,
+                                                               const float* __restrict__ xs, int T, float* y,
+                                                               const float* resid) {
+  extern __shared__ __align__(16) unsigned char gmm_lds[];
+  // [segment of the slice][two chunks][token % 2][lane]: the terms of four blocks
+  float4* terms = reinterpret_cast<float4*>(gmm_lds);
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, W = blockDim.x >> 6;
+  const int n = lane & 15, g = lane >> 4, NB = K >> 5, segs = K / GMM_SEG;
+  const int tiles = (rows + GMM_ROWS - 1) / GMM_ROWS;
+  // as A row n and K group g: the token, and whether this half of K is its block
+  const int xt = 2 * (n >> 2) + (n & 1);
+  const bool xon = xt < T && (g >> 1) == ((n >> 1) & 1);
+  int4 wv[8];
+  uint4 dv[2];
+  v4i_t xv[8];
+  float4* sl = terms + (size_t)W * 8 * 64 + wave * (GMM_MAX * GMM_SEG / 32 / 4);
+  auto load_x = [&](int sg) __attribute__((always_inline)) {
+    const int8_t* xp = xq + (size_t)min(xt, T - 1) * K + sg * GMM_SEG + 16 * g;
+    // (lane: token lane / 4 % 8, blocks 4 (lane % 4) .. + 3)
+    const float4 sc = reinterpret_cast<const float4*>(xs + (size_t)min((lane >> 2) & 7, T - 1) * NB + sg * 16)[lane & 3];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) xv[c] = v4i_t{0, 0, 0, 0};
+    if (xon) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) xv[c] = *reinterpret_cast<const v4i_t*>(xp + 64 * c);
+    }
+    if (lane < 32) sl[(lane & 3) * GMM_MAX + (lane >> 2)] = sc;
+  };
+  auto w_at = [&](int tile, int sg) __attribute__((always_inline)) {
+    return wq + (size_t)min(tile * GMM_ROWS + n, rows - 1) * K + sg * GMM_SEG + 16 * g;
+  };
+  auto d_at = [&](int tile, int sg) __attribute__((always_inline)) {
+    return reinterpret_cast<const uint4*>(wd + (size_t)min(tile * GMM_ROWS + n, rows - 1) * NB + sg * 16);
+  };
+  // the terms of a segment; with next, a chunk's registers take the next segment's loads as soon
+  // as its product is issued
+  auto segment = [&](auto nextc, const int8_t* wn, const uint4* dn) __attribute__((always_inline)) {
+    constexpr bool next = decltype(nextc)::value;
+    float4* tp = terms + (size_t)wave * 8 * 64 + lane;
+#pragma unroll
+    for (int c2 = 0; c2 < 4; ++c2) {
+      float t[2][4];  // [token][block]
+      const float4 sv[2] = {sl[c2 * GMM_MAX + 2 * g], sl[c2 * GMM_MAX + 2 * g + 1]};
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int c = 2 * c2 + u;
+        const v4i_t d = __builtin_amdgcn_mfma_i32_16x16x64_i8(xv[c], v4i_t{wv[c].x, wv[c].y, wv[c].z, wv[c].w},
+                                                              v4i_t{0, 0, 0, 0}, 0, 0, 0);
+        if constexpr (next) wv[c] = *reinterpret_cast<const int4*>(wn + 64 * c);
+        const uint32_t h2[4] = {dv[c >> 2].x, dv[c >> 2].y, dv[c >> 2].z, dv[c >> 2].w};
+        const float w0 = half_bits_to_float((uint16_t)(h2[c & 3] & 0xffffu));
+        const float w1 = half_bits_to_float((uint16_t)(h2[c & 3] >> 16));
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          t[p][2 * u] = ((float)d[p] * w0) * (u ? sv[p].z : sv[p].x);
+          t[p][2 * u + 1] = ((float)d[2 + p] * w1) * (u ? sv[p].w : sv[p].y);
+        }
+      }
+      if constexpr (next)
+        if (c2 & 1) dv[c2 >> 1] = dn[c2 >> 1];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) tp[(c2 * 2 + p) * 64] = make_float4(t[p][0], t[p][1], t[p][2], t[p][3]);
+    }
+  };
+  int tile = blockIdx.x, s0 = 0;
+  const int8_t* wn = w_at(tile, min(wave, segs - 1));
+  const uint4* dn = d_at(tile, min(wave, segs - 1));
+  if (wave < segs) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) wv[c] = *reinterpret_cast<const int4*>(wn + 64 * c);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) dv[i] = dn[i];
+    load_x(wave);
+  }
+  float acc = 0.0f;  // waves 0, 1: token 2 g + wave of row n
+  for (;;) {
+    // what follows: the next slice of the tile, or the first of the next tile
+    const bool last_slice = s0 + W >= segs;
+    const int nt = last_slice ? tile + (int)gridDim.x : tile, ns = last_slice ? 0 : s0 + W;
+    const int sn = ns + wave;
+    wn = w_at(nt, min(sn, segs - 1));
+    dn = d_at(nt, min(sn, segs - 1));
+    if (s0 + wave < segs) {
+      if (nt < tiles && sn < segs)
+        segment(std::true_type{}, wn, dn);
+      else
+        segment(std::false_type{}, wn, dn);
+      if (W < segs && nt < tiles && sn < segs) load_x(sn);
+    }
+    __syncthreads();
+    if (wave < 2) {
+      const float4* tp = terms + wave * 64 + lane;
+      const int ns4 = min(W, segs - s0);
+      // a segment's 16 terms are read while the one before is added
+      float4 va[4], vb[4];
+      auto rd = [&](float4* v, int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = tp[(min(i, ns4 - 1) * 4 + u) * 128];
+      };
+      auto add = [&](const float4* v) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          acc += v[u].x;
+          acc += v[u].y;
+          acc += v[u].z;
+          acc += v[u].w;
+        }
+      };
+      rd(va, 0);
+#pragma unroll 1
+      for (int i = 0; i < ns4; i += 2) {
+        rd(vb, i + 1);
+        add(va);
+        rd(va, i + 2);
+        if (i + 1 < ns4) add(vb);
+      }
+      if (last_slice) {
+        const int t = 2 * g + wave, r = tile * GMM_ROWS + n;
+        if (t < T && r < rows) {
+          const size_t o = (size_t)t * rows + r;
+          y[o] = resid ? resid[o] + acc : acc;
+        }
+        acc = 0.0f;
+      }
+    }
+    if (nt >= tiles) break;
+    __syncthreads();
+    tile = nt;
+    s0 = ns;
   }
 }
 

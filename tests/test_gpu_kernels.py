@@ -148,6 +148,25 @@ def test_q8_gemm_step_edges(native, orc, monkeypatch, rows, k, tokens, nf):
     assert np.array_equal(_bits(y.download(np.float32, rows * tokens).reshape(tokens, rows)), _bits(want))
 
 
+@pytest.mark.parametrize("rows,k,tokens,shift", [(4, 512, 1, 0), (16, 512, 8, 0), (20, 1024, 2, 0), (36, 8192, 5, 0),
+                                                 (20, 8704, 7, 0), (16, 14336, 8, 0), (20, 1024, 3, 2), (20, 1024, 3, 1)])
+def test_q8_gemm_few_tokens(native, orc, rows, k, tokens, shift):
+    """The few-token kernel at its edges: one segment (a wave without products), the most segments of
+    one slice, two slices (9 + 8 and 14 + 14), rows past a 16-row tile, odd token counts; and scales
+    at a 2-byte (shift 1) or 4-byte (2) offset, which it does not take."""
+    rng = np.random.default_rng(rows + 3 * k + tokens)
+    wire = orc.quantize_q8_0_wire(rng.normal(0, 0.02, rows * k).astype(np.float32))
+    q, d = _repack(native, wire, rows, k)
+    pairs = [orc.quantize_q8_0(rng.normal(0, 1 + t % 5, k).astype(np.float32)) for t in range(tokens)]
+    xs, xq = np.stack([p[0] for p in pairs]), np.stack([p[1] for p in pairs])
+    d = np.concatenate([np.zeros(shift, d.dtype), d.ravel()])
+    wq, wd, dxq, dxs, y = _dev(q), _dev(d), _dev(xq), _dev(xs), _buf(rows * tokens * 4)
+    off = getattr(wd.ptr, "value", wd.ptr) + 2 * shift
+    _ok(native.camelid_hip_q8_0_gemm(wq.ptr, off, rows, k, dxq.ptr, dxs.ptr, tokens, y.ptr, None, None))
+    want = np.stack([orc.q8_0_gemv(wire, rows, k, xs[t], xq[t]) for t in range(tokens)])
+    assert np.array_equal(_bits(y.download(np.float32, rows * tokens).reshape(tokens, rows)), _bits(want))
+
+
 @pytest.mark.parametrize("rows,k", [(32000, 2048), (128256, 3072)])
 def test_q8_gemm_bit_exact_large(native, orc, rows, k):
     """The sweep's two largest shapes (TinyLlama's and Llama-3.2-3B's lm_head widths) at the
