@@ -1381,12 +1381,19 @@ uint32_t q6m_tokens(uint32_t K) {
   return t;
 }
 
+constexpr uint32_t Q4K_MM_MIN = 1, Q6K_MM_MIN = 1;
+
 // A K-quant projection over T tokens with Q8_K activation rows (kd [T][k/256], kq [T][k]):
 // y[t * ldy + row] (+ resid, same stride).  Q4_K: the matrix-core GEMM; Q6_K: for more than
 // Q6M_MAX tokens the class-major GEMM (needs m.w2 and xt, cm::q6g_act_bytes(T, k) bytes for
 // the class-major copy of kq) or else the sparse-MFMA GEMM, for fewer the multi-token GEMV.
 void launch_kgemm(const KMat& m, uint32_t T, const float* kd, const int8_t* kq, float* y, uint32_t ldy,
                   const float* resid, hipStream_t s, int8_t* xt) {
+  if (m.quant == CAMELID_Q4_K && T >= Q4K_MM_MIN && T <= (uint32_t)cm::Q4X_MAX) {  // a few tokens, the matrix cores
+    CM_LAUNCH(cm::k_gemv_q4k_mm, dim3(cm::q4x_grid((int)m.rows)), dim3(cm::Q4X_W * 64), cm::Q4X_LDS, s, m.a, m.b,
+              (int)m.rows, (int)m.k, kd, kq, (int)T, y, (int)ldy, resid);
+    return;
+  }
   if (m.quant == CAMELID_Q4_K && T <= (uint32_t)cm::Q4M_MAX) {  // a few tokens (verify)
     uint32_t tt = T;
     while (tt > 1 && cm::gemv_q4k_multi_lds_bytes((int)m.k, (int)tt) > 65536) --tt;
@@ -1428,6 +1435,18 @@ void launch_kgemm(const KMat& m, uint32_t T, const float* kd, const int8_t* kq, 
               dim3(cm::G6_NT), 0, s, m.a, m.b, m.sc, m.d, (int)m.rows, (int)m.k, kd, kq, (int)T, y, (int)ldy, resid);
     return;
   }
+  if (T >= Q6K_MM_MIN) {  // the matrix cores
+    const dim3 grid(cm::q6x_grid((int)m.rows)), block(cm::Q6X_W * 64);
+    switch ((T + 1) / 2) {
+#define CM_Q6X(NP)                                                                                              \
+  case NP:                                                                                                      \
+    CM_LAUNCH(cm::k_gemv_q6k_mm<NP>, grid, block, cm::q6x_lds_bytes(NP), s, m.a, m.b, m.sc, m.d, (int)m.rows,   \
+              (int)m.k, kd, kq, (int)T, y, (int)ldy, resid);                                                    \
+    return;
+      CM_Q6X(1) CM_Q6X(2) CM_Q6X(3) CM_Q6X(4)
+#undef CM_Q6X
+    }
+  }
   const uint32_t tt = q6m_tokens(m.k), nsb = m.k / 256;
   for (uint32_t t0 = 0; t0 < T; t0 += tt) {
     const uint32_t n = std::min(tt, T - t0);
@@ -1444,7 +1463,7 @@ void launch_kgemm(const KMat& m, uint32_t T, const float* kd, const int8_t* kq, 
 constexpr int GEMM_BIG_TILES = 288;
 void launch_gemm(const Q8Mat& m, uint32_t T, const int8_t* xq, const float* xs, float* y, const float* resid,
                  hipStream_t s) {
-  if (T <= (uint32_t)cm::GMT_MAX && m.k <= 8192) {  // one or two tokens
+  if (T <= (uint32_t)cm::GMT_MAX && m.k <= 8192) {  // up to three tokens
     const uint32_t grid = (m.rows + cm::GMT_ROWS - 1) / cm::GMT_ROWS;
     const size_t lds = cm::gemv_multi_lds_bytes((int)m.k, (int)T);
     switch (m.k) {

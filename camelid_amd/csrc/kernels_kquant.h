@@ -1040,6 +1040,177 @@ __global__ __launch_bounds__(KQ_NT) void k_gemv_q6k_multi(const uint8_t* __restr
 }
 
 // ---------------------------------------------------------------------------
+// The same for 2 NP tokens at most on the matrix cores (speculative verify, short prefill chunks).
+// The Q6_K dot needs, per superblock, its eight class sums aux[l] = sum over p = l (mod 8) of
+// sc[p / 16] * (w[p] - 32) * q8[p].  The products sc (w - 32) (13 bits and a sign) are formed from
+// the weights as they lie in memory, two to a v_pk_mad_u16, and split into signed bytes as
+// 256 h + lo; they are the B operand of v_mfma_i32_16x16x64_i8 (lane (n, g): one 16-value scale
+// group of row n per product).  The 16 rows of the A operand are two tokens' eight classes: a row
+// holds a token's quants with every byte of another class masked to zero, so one product per plane
+// gives 16 rows x 2 tokens x 8 classes, exactly, and 64 weights per lane take ~160 VALU operations
+// for all tokens where k_gemv_q6k_multi takes ~130 for each.
+// Workgroup: 16 rows; each wave one superblock of the slice, its next weights on their way
+// meanwhile; the terms (d * y.d) * aux go to LDS, where one thread per (row, token, class) adds
+// them in superblock order; eight lanes then meet for the left fold from -0.0.  Rows of more than
+// Q6X_W superblocks go in slices, the class sums carried along.
+// K % 256 == 0.  Dynamic LDS: q6x_lds_bytes(NP).
+constexpr int Q6X_W = 16;  // waves of a workgroup = superblocks of a slice
+constexpr int Q6X_ROWS = 16;
+constexpr int Q6X_CUS = 256;  // one workgroup of 16 waves per CU
+inline size_t q6x_lds_bytes(int np) { return (size_t)Q6X_W * np * (64 * 16 + 512); }
+inline int q6x_grid(int rows) { return rows > Q6X_ROWS * Q6X_CUS ? Q6X_CUS : (rows + Q6X_ROWS - 1) / Q6X_ROWS; }
+
+typedef unsigned short q6x_u2 __attribute__((ext_vector_type(2)));
+
+template <int NP>
+__global__ __launch_bounds__(Q6X_W * 64) void k_gemv_q6k_mm(const uint8_t* __restrict__ ql,
+                                                            const uint8_t* __restrict__ qh,
+                                                            const int8_t* __restrict__ scl,
+                                                            const uint16_t* __restrict__ dw, int rows, int K,
+                                                            const float* __restrict__ yd,
+                                                            const int8_t* __restrict__ yq, int T, float* y, int ldy,
+                                                            const float* resid) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int NSB = K >> 8, tiles = (rows + Q6X_ROWS - 1) / Q6X_ROWS;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int n = lane & 15, g = lane >> 4;
+  float* terms = reinterpret_cast<float*>(smem);  // [wave][token pair][lane][4 classes]
+  int4* xl = reinterpret_cast<int4*>(smem + (size_t)Q6X_W * NP * 64 * 16) + wave * NP * 32;  // [token][16 pieces]
+  // as A row n: token n / 8 of the pair, class n % 8 (bytes n % 8 and 8 + n % 8 of 16)
+  const int cbyte = (int)(0xffu << (8 * (n & 3)));
+  const int m0 = (n & 4) ? 0 : cbyte, m1 = (n & 4) ? cbyte : 0;
+  struct unit {
+    uint4 l0, l1, hh;
+    uint2 sc;
+    uint32_t d;
+  };
+  auto load = [&](unit& w, int tile, int s) __attribute__((always_inline)) {
+    const size_t row = (size_t)min(tile * Q6X_ROWS + n, rows - 1);
+    const uint8_t* a = ql + row * (K >> 1) + s * 128 + (g >> 1) * 64 + (g & 1) * 16;
+    w.l0 = *reinterpret_cast<const uint4*>(a);
+    w.l1 = *reinterpret_cast<const uint4*>(a + 32);
+    w.hh = *reinterpret_cast<const uint4*>(qh + row * (K >> 2) + s * 64 + (g >> 1) * 32 + (g & 1) * 16);
+    w.sc = *reinterpret_cast<const uint2*>(scl + (row * NSB + s) * 16 + (g >> 1) * 8);
+    w.d = dw[row * NSB + s];
+  };
+  // a superblock's quants: lanes of token lane / 8 (< 2 NP), two 16-byte pieces each; and this lane's scales
+  int4 xr[2];
+  float xd[NP];
+  auto load_x = [&](int s) __attribute__((always_inline)) {
+    const int4* p = reinterpret_cast<const int4*>(yq + (size_t)min(lane >> 3, T - 1) * K + s * 256) + 2 * (lane & 7);
+    xr[0] = p[0];
+    xr[1] = p[1];
+#pragma unroll
+    for (int j = 0; j < NP; ++j) xd[j] = yd[(size_t)min(2 * j + (g >> 1), T - 1) * NSB + s];
+  };
+  auto put_x = [&]() __attribute__((always_inline)) {
+    if (lane < 16 * NP) {
+      xl[2 * lane] = xr[0];
+      xl[2 * lane + 1] = xr[1];
+    }
+    // (this wave's own LDS)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  auto product = [&](const unit& w) __attribute__((always_inline)) {
+    const uint32_t M4 = 0x0f0f0f0fu, MH = 0x30303030u;
+    const uint32_t L0[4] = {w.l0.x, w.l0.y, w.l0.z, w.l0.w}, L1[4] = {w.l1.x, w.l1.y, w.l1.z, w.l1.w};
+    const uint32_t HH[4] = {w.hh.x, w.hh.y, w.hh.z, w.hh.w};
+    v4i_t ch[NP], cl[NP];
+#pragma unroll
+    for (int j = 0; j < NP; ++j) ch[j] = cl[j] = v4i_t{0, 0, 0, 0};
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {  // scale group 8 (g / 2) + g % 2 + 2 kk, positions 16 times that on
+      const uint32_t scw = (kk < 2 ? w.sc.x : w.sc.y) >> (16 * (kk & 1));
+      const int sc = (int)(int8_t)(scw >> (8 * (g & 1)));
+      const unsigned short s1 = (unsigned short)sc, c1 = (unsigned short)(128 - 32 * sc);
+      const q6x_u2 s2 = {s1, s1}, c2 = {c1, c1};
+      v4i_t bh, bl;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t lq = (kk & 1) ? L1[u] : L0[u];
+        const uint32_t lo = (kk < 2) ? (lq & M4) : ((lq >> 4) & M4);
+        const uint32_t hi = (kk == 0 ? HH[u] << 4 : kk == 1 ? HH[u] << 2 : kk == 2 ? HH[u] : HH[u] >> 2) & MH;
+        const uint32_t v = lo | hi, ev = v & 0x00ff00ffu, ov = (v >> 8) & 0x00ff00ffu;
+        // sc (w - 32) + 128 per 16 bits: the high byte is h, the low byte lo + 128
+        const q6x_u2 pe = __builtin_bit_cast(q6x_u2, ev) * s2 + c2, po = __builtin_bit_cast(q6x_u2, ov) * s2 + c2;
+        const uint32_t e = __builtin_bit_cast(uint32_t, pe), o = __builtin_bit_cast(uint32_t, po);
+        bh[u] = (int)__builtin_amdgcn_perm(o, e, 0x07030501u);
+        bl[u] = (int)(__builtin_amdgcn_perm(o, e, 0x06020400u) ^ 0x80808080u);
+      }
+#pragma unroll
+      for (int j = 0; j < NP; ++j) {
+        const int4 x = xl[(2 * j + (n >> 3)) * 16 + (g >> 1) * 8 + (g & 1) + 2 * kk];
+        const v4i_t a = {x.x & m0, x.y & m1, x.z & m0, x.w & m1};
+        ch[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, bh, ch[j], 0, 0, 0);
+        cl[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, bl, cl[j], 0, 0, 0);
+      }
+    }
+    // this lane: row n, token 2 j + g / 2, classes 4 (g % 2) ..
+    const float dsb = half_bits_to_float((uint16_t)w.d);
+#pragma unroll
+    for (int j = 0; j < NP; ++j) {
+      const float d = dsb * xd[j];
+      float t[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) t[i] = d * (float)(ch[j][i] * 256 + cl[j][i]);
+      reinterpret_cast<float4*>(terms)[(wave * NP + j) * 64 + lane] = make_float4(t[0], t[1], t[2], t[3]);
+    }
+  };
+  // this thread's chain: token pair tid / 256, token of the pair, row, class; and its term's place
+  const int cj = tid >> 8, ct = 2 * cj + ((tid >> 7) & 1), cr = (tid >> 3) & 15, cc = tid & 7;
+  const float* chain = terms + (cj * 64 + cr + 16 * (2 * ((tid >> 7) & 1) + (cc >> 2))) * 4 + (cc & 3);
+  const bool folds = tid < NP * 256;
+  float sum = 0.0f;
+
+  int tile = blockIdx.x, s0 = 0;
+  unit w;
+  load(w, tile, min(wave, NSB - 1));
+  load_x(min(wave, NSB - 1));
+  put_x();
+  for (;;) {
+    // what follows: the next slice of the tile, or the first of the next tile
+    const bool last = s0 + Q6X_W >= NSB;
+    const int nt = last ? tile + (int)gridDim.x : tile, ns = last ? 0 : s0 + Q6X_W;
+    unit wn = w;
+    if (nt < tiles) load(wn, nt, min(ns + wave, NSB - 1));
+    if (s0 + wave < NSB) product(w);
+    if (NSB > Q6X_W && nt < tiles) load_x(min(ns + wave, NSB - 1));
+    __syncthreads();
+    if (folds) {
+      const int cnt = min(Q6X_W, NSB - s0);
+      if (cnt == Q6X_W) {
+        float v[Q6X_W];
+#pragma unroll
+        for (int i = 0; i < Q6X_W; ++i) v[i] = chain[i * NP * 256];
+#pragma unroll
+        for (int i = 0; i < Q6X_W; ++i) sum += v[i];
+      } else {
+        for (int i = 0; i < cnt; ++i) sum += chain[i * NP * 256];
+      }
+      if (last) {
+        float acc = -0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc += __shfl(sum, (lane & ~7) + i);
+        const int row = tile * Q6X_ROWS + cr;
+        if (cc == 0 && ct < T && row < rows) {
+          const size_t o = (size_t)ct * ldy + row;
+          y[o] = resid ? resid[o] + acc : acc;
+        }
+        sum = 0.0f;
+      }
+    }
+    if (nt >= tiles) break;
+    __syncthreads();
+    if (NSB > Q6X_W) put_x();
+    w = wn;
+    tile = nt;
+    s0 = ns;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Q6_K GEMM for prefill chunks: each (token, row) is k_gemv_q6k's result (the Q6_K decode dot
 // of inference.rs:19148-19195):  aux[l] = sum over positions p = l (mod 8) of
 // sc[p/16] * q8[p] * w[p] per superblock (exact integers), sums[l] += (f16(d) * y.d) * aux[l]
@@ -1522,6 +1693,185 @@ __global__ __launch_bounds__(KQ_NT) void k_gemv_q4k_multi(const uint8_t* __restr
       const size_t o = (size_t)t * ldy + r;
       y[o] = resid ? resid[o] + acc : acc;
     }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The same for 1 <= T <= Q4X_MAX tokens on the matrix cores.  With each 6-bit sub-block scale split
+// as sc = 8 sh + sl (as k_gemm_q4k), a superblock's sums are three K = 256 dots of signed bytes,
+// sumi = 8 (sh q . x) + (sl q . x) and prod = mn . x, from v_mfma_i32_16x16x64_i8: the weights are
+// the B operand as they lie in memory (lane (n, g): 32 bytes of row n, sub-blocks 2 g and 2 g + 1,
+// four products of 16 positions), and the 16 rows of the A operand are 8 tokens in each of two
+// superblocks, a token's row being zero in the other superblock's products (read from a zero block
+// in LDS), so that every lane's four results are wanted.
+// Workgroup: 16 rows, Q4X_W waves of two superblocks each, the next ones' weights on their way
+// meanwhile; terms through LDS, one thread per (row, token) folds them in superblock order; rows
+// of more than 2 Q4X_W superblocks in slices.  k_gemv_q4k_multi's VALU work is per token, this
+// one's is not.
+// K % 256 == 0.  Dynamic LDS: Q4X_LDS.
+constexpr int Q4X_MAX = 8;
+constexpr int Q4X_W = 8;  // waves
+constexpr int Q4X_ROWS = 16;
+constexpr int Q4X_RESIDENT = 512;  // two workgroups per CU
+constexpr size_t Q4X_LDS = Q4X_W * (4 * 64 * 16 + 2 * Q4X_MAX * 256) + 64;
+inline int q4x_grid(int rows) {
+  const int tiles = (rows + Q4X_ROWS - 1) / Q4X_ROWS;
+  return tiles < Q4X_RESIDENT ? tiles : Q4X_RESIDENT;
+}
+
+__global__ __launch_bounds__(Q4X_W * 64, 4) void k_gemv_q4k_mm(const uint8_t* __restrict__ nib,
+                                                               const uint8_t* __restrict__ hdr, int rows, int K,
+                                                               const float* __restrict__ yd,
+                                                               const int8_t* __restrict__ yq, int T, float* y, int ldy,
+                                                               const float* resid) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int NSB = K >> 8, tiles = (rows + Q4X_ROWS - 1) / Q4X_ROWS;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int n = lane & 15, g = lane >> 4;
+  float4* terms = reinterpret_cast<float4*>(smem);  // [wave][result][lane]
+  int4* xl = reinterpret_cast<int4*>(smem + Q4X_W * 4 * 64 * 16) + wave * 2 * Q4X_MAX * 16;  // [superblock][token][16]
+  int4* zero = reinterpret_cast<int4*>(smem + Q4X_W * (4 * 64 * 16 + 2 * Q4X_MAX * 256));
+  // as A row n: token n % 8 of superblock n / 8
+  const int4* xa0 = n < 8 ? xl + n * 16 + 4 * g : zero;
+  const int4* xa1 = n < 8 ? zero : xl + n * 16 + 4 * g;
+  struct unit {
+    uint4 a[2], h;  // 32 bytes of nibbles, the header
+  };
+  auto load = [&](unit& w, int tile, int s) __attribute__((always_inline)) {
+    const size_t row = (size_t)min(tile * Q4X_ROWS + n, rows - 1);
+    const int sc = min(s, NSB - 1);
+    const uint4* p = reinterpret_cast<const uint4*>(nib + row * (K >> 1)) + sc * 8 + 2 * g;
+    w.a[0] = p[0];
+    w.a[1] = p[1];
+    w.h = *(reinterpret_cast<const uint4*>(hdr + row * NSB * 16) + sc);
+  };
+  // both superblocks' quants (lane: token lane / 8, two 16-byte pieces) and this lane's scales
+  int4 xr[2][2];
+  float xd[4];
+  auto load_x = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int4* p = reinterpret_cast<const int4*>(yq + (size_t)min(lane >> 3, T - 1) * K) +
+                      min(s + b, NSB - 1) * 16 + 2 * (lane & 7);
+      xr[b][0] = p[0];
+      xr[b][1] = p[1];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      xd[i] = yd[(size_t)min(4 * (g & 1) + i, T - 1) * NSB + min(s + (g >> 1), NSB - 1)];
+  };
+  auto put_x = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) xl[b * Q4X_MAX * 16 + 2 * lane + j] = xr[b][j];
+    // (this wave's own LDS)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  typedef unsigned short u2_t __attribute__((ext_vector_type(2)));
+  auto product = [&](const unit (&w)[2]) __attribute__((always_inline)) {
+    const uint32_t K1 = 0x3f3f3f3fu, K2 = 0x0f0f0f0fu, K3 = 0x03030303u;
+    v4i_t ch = {0, 0, 0, 0}, cl = {0, 0, 0, 0}, cm = {0, 0, 0, 0};
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const uint4 hd = w[b].h;
+      const uint32_t scw = ((g < 2) ? (hd.y & K1) : ((hd.w & K2) | (((hd.y >> 6) & K3) << 4))) >> (16 * (g & 1));
+      const uint32_t mnw = ((g < 2) ? (hd.z & K1) : (((hd.w >> 4) & K2) | (((hd.z >> 6) & K3) << 4))) >> (16 * (g & 1));
+#pragma unroll
+      for (int hi = 0; hi < 2; ++hi) {  // sub-block 2 g + hi
+        const uint32_t sc = (scw >> (8 * hi)) & 0xffu, mn = ((mnw >> (8 * hi)) & 0xffu) * 0x01010101u;
+        const unsigned short sh = (unsigned short)(sc >> 3), sl = (unsigned short)(sc & 7u);
+        const u2_t sh2 = {sh, sh}, sl2 = {sl, sl};
+        const v4i_t bm = {(int)mn, (int)mn, (int)mn, (int)mn};
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {  // its positions 16 p ..
+          const uint4 a4 = w[b].a[p];
+          const uint32_t A[4] = {a4.x, a4.y, a4.z, a4.w};
+          v4i_t bh, bl;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            // bytes <= 15 * 7: no carry between them
+            const u2_t q = __builtin_bit_cast(u2_t, (hi ? A[u] >> 4 : A[u]) & K2);
+            bh[u] = __builtin_bit_cast(int, (u2_t)(q * sh2));
+            bl[u] = __builtin_bit_cast(int, (u2_t)(q * sl2));
+          }
+          const int4 x4 = (b ? xa1 : xa0)[2 * hi + p];
+          const v4i_t x = {x4.x, x4.y, x4.z, x4.w};
+          ch = __builtin_amdgcn_mfma_i32_16x16x64_i8(x, bh, ch, 0, 0, 0);
+          cl = __builtin_amdgcn_mfma_i32_16x16x64_i8(x, bl, cl, 0, 0, 0);
+          cm = __builtin_amdgcn_mfma_i32_16x16x64_i8(x, bm, cm, 0, 0, 0);
+        }
+      }
+    }
+    // this lane: row n, superblock g / 2, tokens 4 (g % 2) ..
+    const uint32_t dd = g < 2 ? w[0].h.x : w[1].h.x;
+    const float dw = half_bits_to_float((uint16_t)(dd & 0xffffu)), dmw = half_bits_to_float((uint16_t)(dd >> 16));
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      terms[(wave * 4 + i) * 64 + lane] =
+          make_float4(-(xd[i] * dmw), (float)cm[i], xd[i] * dw, (float)(ch[i] * 8 + cl[i]));
+  };
+  // this thread's chain (the first 128): row and token; and its terms' place
+  const int cr = tid & 15, ct = (tid >> 4) & 7;
+  const float4* chain = terms + (ct & 3) * 64 + cr + 16 * (ct >> 2);
+  float acc = 0.0f;
+
+  int tile = blockIdx.x, s0 = 0;
+  unit w[2];
+  load(w[0], tile, 2 * wave);
+  load(w[1], tile, 2 * wave + 1);
+  load_x(2 * wave);
+  if (tid < 4) zero[tid] = make_int4(0, 0, 0, 0);
+  put_x();
+  __syncthreads();
+  for (;;) {
+    // what follows: the next slice of the tile, or the first of the next tile
+    const bool last = s0 + 2 * Q4X_W >= NSB;
+    const int nt = last ? tile + (int)gridDim.x : tile, ns = last ? 0 : s0 + 2 * Q4X_W;
+    unit wn[2] = {w[0], w[1]};
+    if (nt < tiles) {
+      load(wn[0], nt, ns + 2 * wave);
+      load(wn[1], nt, ns + 2 * wave + 1);
+    }
+    if (s0 + 2 * wave < NSB) product(w);
+    if (NSB > 2 * Q4X_W && nt < tiles) load_x(ns + 2 * wave);
+    __syncthreads();
+    if (tid < 16 * Q4X_MAX) {
+      const int cnt = min(2 * Q4X_W, NSB - s0);
+      auto add = [&](const float4& v) __attribute__((always_inline)) {
+        acc = fmaf(v.x, v.y, acc);
+        acc = fmaf(v.z, v.w, acc);
+      };
+      if (cnt == 2 * Q4X_W) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          float4 v[Q4X_W];
+#pragma unroll
+          for (int i = 0; i < Q4X_W; ++i) v[i] = chain[((Q4X_W * h + i) >> 1) * 256 + 32 * (i & 1)];
+#pragma unroll
+          for (int i = 0; i < Q4X_W; ++i) add(v[i]);
+        }
+      } else {
+        for (int i = 0; i < cnt; ++i) add(chain[(i >> 1) * 256 + 32 * (i & 1)]);
+      }
+      if (last) {
+        const int row = tile * Q4X_ROWS + cr;
+        if (ct < T && row < rows) {
+          const size_t o = (size_t)ct * ldy + row;
+          y[o] = resid ? resid[o] + acc : acc;
+        }
+        acc = 0.0f;
+      }
+    }
+    if (nt >= tiles) break;
+    __syncthreads();
+    if (NSB > 2 * Q4X_W) put_x();
+    w[0] = wn[0];
+    w[1] = wn[1];
+    tile = nt;
+    s0 = ns;
   }
 }
 

@@ -718,6 +718,35 @@ def test_kquant_gemm_bit_exact(native, orc, quant, rows, k, T, ldy):
             assert np.array_equal(_bits(want), _bits(orc.kquant_gemv(quant, wire, rows, k, ydh[t], yqh[t])))
 
 
+@pytest.mark.parametrize("quant,rows,k,T", [(1, 3, 256, 4), (1, 16, 768, 8), (1, 17, 4096, 5), (1, 31, 4352, 7),
+                                            (1, 8209, 512, 6), (1, 20, 16384, 8), (2, 3, 256, 4), (2, 16, 3840, 8),
+                                            (2, 17, 4096, 5), (2, 31, 4352, 7), (2, 4113, 512, 6), (2, 20, 16384, 8),
+                                            (1, 40, 8448, 2), (2, 40, 8448, 2), (1, 33, 2048, 3), (2, 33, 2048, 3)])
+def test_kquant_few_tokens_edges(native, orc, quant, rows, k, T):
+    """The few-token kernels at their edges: one superblock, an odd number of them, a slice and one
+    superblock more, several slices; rows short of, at and past a 16-row tile and more tiles than
+    resident workgroups; odd token counts; scales and quants over their whole ranges (Q6_K: scale
+    products of +4096 and -4064 in rows 0 and 1).  Every value is the CPU dot's, bit for bit."""
+    rng = np.random.default_rng(rows + 3 * k + T + quant)
+    wire = _kquant_wire(orc, rng, quant, rows, k)
+    if quant == 2:
+        ends = wire.reshape(rows, k // 256, 210)
+        ends[0, :, :192], ends[0, :, 192:208] = 0, 0x80
+        ends[1, :, :192], ends[1, :, 192:208] = 0, 0x7F
+    a, b, sc, d = _kquant_planes(native, quant, wire, rows, k)
+    x = rng.normal(0, 1, (T, k)).astype(np.float32)
+    x[0] = -1.0
+    x[0, ::256] = 1.0  # (quants of -127 and +127)
+    yds, yqs = zip(*(orc.quantize_q8_k(x[t]) for t in range(T)))
+    ydh, yqh = np.stack(yds).astype(np.float32), np.stack(yqs).astype(np.int8)
+    yd, yq, y = _dev(ydh), _dev(yqh), _buf(T * rows * 4)
+    _ok(native.camelid_hip_kquant_gemm(quant, a.ptr, b.ptr, sc.ptr, d.ptr, rows, k, T, yd.ptr, yq.ptr, y.ptr, rows,
+                                       None, None))
+    got = y.download(np.float32, T * rows).reshape(T, rows)
+    for t in range(T):
+        assert np.array_equal(_bits(got[t]), _bits(orc.kquant_gemv(quant, wire, rows, k, ydh[t], yqh[t]))), f"token {t}"
+
+
 @pytest.mark.parametrize("case", ["min", "max", "mixed"])
 def test_q6k_gemm_extreme_products(native, orc, case):
     """Q6_K chunk GEMM at the ends of its integer range: scaled weights sc * w of +4096 (sc =
