@@ -1480,9 +1480,12 @@ void launch_gemm(const Q8Mat& m, uint32_t T, const int8_t* xq, const float* xs, 
   // a few tokens: weights streamed once by GEMV-shaped workgroups (16-byte loads of the scales too)
   if (T <= (uint32_t)cm::GMM_MAX && m.k % cm::GMM_SEG == 0 &&
       ((reinterpret_cast<uintptr_t>(m.d) | reinterpret_cast<uintptr_t>(xs)) & 15) == 0) {
-    CM_LAUNCH(cm::k_gemv_mm, dim3(cm::gemv_mm_grid((int)m.rows, (int)m.k)),
-              dim3(64 * cm::gemv_mm_waves((int)m.k)), cm::gemv_mm_lds_bytes((int)m.k), s, m.q, m.d, (int)m.rows,
-              (int)m.k, xq, xs, (int)T, y, resid);
+    const dim3 grid(cm::gemv_mm_grid((int)m.rows, (int)m.k)), block(64 * cm::gemv_mm_waves((int)m.k));
+    const size_t lds = cm::gemv_mm_lds_bytes((int)m.k);
+    if (cm::gemv_mm_sliced((int)m.k))
+      CM_LAUNCH(cm::k_gemv_mm<true>, grid, block, lds, s, m.q, m.d, (int)m.rows, (int)m.k, xq, xs, (int)T, y, resid);
+    else
+      CM_LAUNCH(cm::k_gemv_mm<false>, grid, block, lds, s, m.q, m.d, (int)m.rows, (int)m.k, xq, xs, (int)T, y, resid);
     return;
   }
   // CAMELID_HIP_GEMM_NF=1 / 2 forces the 32 / 64 tiles

@@ -205,6 +205,7 @@ inline int gemv_mm_waves(int K) {
   const int w = (segs + slices - 1) / slices;
   return w < 2 ? 2 : w;
 }
+inline bool gemv_mm_sliced(int K) { return K / GMM_SEG > GMM_WAVES; }
 // per wave: the terms of a segment, then its activation scales [two chunks][token][block]
 constexpr int GMM_WAVE_LDS = 8 * 64 * 16 + GMM_MAX * (GMM_SEG / 32) * 4;
 inline size_t gemv_mm_lds_bytes(int K) { return (size_t)gemv_mm_waves(K) * GMM_WAVE_LDS; }
@@ -214,11 +215,13 @@ inline int gemv_mm_grid(int rows, int K) {
   return tiles < res ? tiles : res;
 }
 
+// SLICED: rows of more than one slice (gemv_mm_sliced(K)).
+template <bool SLICED>
 __global__ __launch_bounds__(GMM_WAVES * 64) void k_gemv_mm(const int8_t* __restrict__ wq,
-                                                               const uint16_t* __restrict__ wd, int rows, int K,
-                                                               const int8_t* __restrict__ xq,
-                                                               const float* __restrict__ xs, int T, float* y,
-                                                               const float* resid) {
+                                                            const uint16_t* __restrict__ wd, int rows, int K,
+                                                            const int8_t* __restrict__ xq,
+                                                            const float* __restrict__ xs, int T, float* y,
+                                                            const float* resid) {
   extern __shared__ __align__(16) unsigned char gmm_lds[];
   // [segment of the slice][two chunks][token % 2][lane]: the terms of four blocks
   float4* terms = reinterpret_cast<float4*>(gmm_lds);
@@ -249,6 +252,12 @@ __global__ __launch_bounds__(GMM_WAVES * 64) void k_gemv_mm(const int8_t* __rest
   };
   auto d_at = [&](int tile, int sg) __attribute__((always_inline)) {
     return reinterpret_cast<const uint4*>(wd + (size_t)min(tile * GMM_ROWS + n, rows - 1) * NB + sg * 16);
+  };
+  auto load_w = [&](const int8_t* wn, const uint4* dn) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) wv[c] = *reinterpret_cast<const int4*>(wn + 64 * c);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) dv[i] = dn[i];
   };
   // the terms of a segment; with next, a chunk's registers take the next segment's loads as soon
   // as its product is issued
@@ -284,27 +293,27 @@ __global__ __launch_bounds__(GMM_WAVES * 64) void k_gemv_mm(const int8_t* __rest
   const int8_t* wn = w_at(tile, min(wave, segs - 1));
   const uint4* dn = d_at(tile, min(wave, segs - 1));
   if (wave < segs) {
-#pragma unroll
-    for (int c = 0; c < 8; ++c) wv[c] = *reinterpret_cast<const int4*>(wn + 64 * c);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) dv[i] = dn[i];
+    load_w(wn, dn);
     load_x(wave);
   }
   float acc = 0.0f;  // waves 0, 1: token 2 g + wave of row n
   for (;;) {
     // what follows: the next slice of the tile, or the first of the next tile
-    const bool last_slice = s0 + W >= segs;
+    const bool last_slice = !SLICED || s0 + W >= segs;
     const int nt = last_slice ? tile + (int)gridDim.x : tile, ns = last_slice ? 0 : s0 + W;
     const int sn = ns + wave;
+    const bool more = nt < tiles && sn < segs;  // this wave has work there
     wn = w_at(nt, min(sn, segs - 1));
     dn = d_at(nt, min(sn, segs - 1));
     if (s0 + wave < segs) {
-      if (nt < tiles && sn < segs)
+      if (more)
         segment(std::true_type{}, wn, dn);
       else
         segment(std::false_type{}, wn, dn);
-      if (W < segs && nt < tiles && sn < segs) load_x(sn);
+    } else if (SLICED && more) {  // idle in a short last slice, not in what follows
+      load_w(wn, dn);
     }
+    if (SLICED && more) load_x(sn);
     __syncthreads();
     if (wave < 2) {
       const float4* tp = terms + wave * 64 + lane;

@@ -167,6 +167,26 @@ def test_q8_gemm_few_tokens(native, orc, rows, k, tokens, shift):
     assert np.array_equal(_bits(y.download(np.float32, rows * tokens).reshape(tokens, rows)), _bits(want))
 
 
+@pytest.mark.parametrize("rows,k,tokens", [(4112, 8704, 5), (5120, 13824, 8), (8192, 9728, 1), (5120, 17408, 4)])
+def test_q8_gemm_few_tokens_short_last_slice(native, orc, rows, k, tokens):
+    """The few-token kernel where a row's K goes in two or three slices, the last one short, and a
+    workgroup takes several row tiles: waves idle in the last slice of a tile have work in the
+    first slice of the next.  Every row, bit for bit, also onto a residual in place."""
+    from camelid_amd.model import synth_q8_0
+    rng = np.random.default_rng(rows + 3 * k + tokens)
+    wire = synth_q8_0(f"slices{rows}x{k}", 2, rows, k, 0.02)
+    q, d = _repack(native, wire, rows, k)
+    pairs = [orc.quantize_q8_0(rng.normal(0, 1 + t % 5, k).astype(np.float32)) for t in range(tokens)]
+    xs, xq = np.stack([p[0] for p in pairs]), np.stack([p[1] for p in pairs])
+    resid = rng.normal(0, 1, (tokens, rows)).astype(np.float32)
+    wq, wd, dxq, dxs, dres, y = _dev(q), _dev(d), _dev(xq), _dev(xs), _dev(resid), _buf(rows * tokens * 4)
+    want = np.stack([orc.q8_0_gemv(wire, rows, k, xs[t], xq[t]) for t in range(tokens)])
+    _ok(native.camelid_hip_q8_0_gemm(wq.ptr, wd.ptr, rows, k, dxq.ptr, dxs.ptr, tokens, y.ptr, None, None))
+    assert np.array_equal(_bits(y.download(np.float32, rows * tokens).reshape(tokens, rows)), _bits(want))
+    _ok(native.camelid_hip_q8_0_gemm(wq.ptr, wd.ptr, rows, k, dxq.ptr, dxs.ptr, tokens, dres.ptr, dres.ptr, None))
+    assert np.array_equal(_bits(dres.download(np.float32, rows * tokens).reshape(tokens, rows)), _bits(resid + want))
+
+
 @pytest.mark.parametrize("rows,k", [(32000, 2048), (128256, 3072)])
 def test_q8_gemm_bit_exact_large(native, orc, rows, k):
     """The sweep's two largest shapes (TinyLlama's and Llama-3.2-3B's lm_head widths) at the
