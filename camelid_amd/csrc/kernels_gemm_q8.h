@@ -98,7 +98,9 @@ __global__ __launch_bounds__(GM_NT, 4) void k_gemm_q8(const int8_t* __restrict__
   __shared__ __align__(16) gm_i4 sb[2][C::CH][C::PL];
   __shared__ __align__(16) float sx[2][SB][C::TR];
   __shared__ __align__(16) float2 sw[2][SB][C::TR];
-  __shared__ int sinf;  // a staged weight scale was infinite
+  // bit b: a weight scale staged into buffer b was infinite.  A step tests its own buffer's bit while
+  // the other one's may be set, so all waves of the workgroup leave the first loop at the same step.
+  __shared__ uint32_t sinf;
   const int NB = K >> 5, nsteps = (NB + SB - 1) / SB;
   const int ntt = (T + C::TR - 1) / C::TR, tiles = gm_tiles(N, T, M), per = (tiles + 7) >> 3;
   const int L = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
@@ -146,7 +148,7 @@ __global__ __launch_bounds__(GM_NT, 4) void k_gemm_q8(const int8_t* __restrict__
     __builtin_memcpy(&h, &rw, 2);
     const float w = (float)h;
     sw[buf][sblk][srow] = make_float2(w, -GM_MAGIC_F * w);
-    if ((rw & 0x7fffu) == 0x7c00u) sinf = 1;
+    if ((rw & 0x7fffu) == 0x7c00u) atomicOr(&sinf, 1u << buf);
   };
 
   float acc[R];
@@ -200,10 +202,14 @@ __global__ __launch_bounds__(GM_NT, 4) void k_gemm_q8(const int8_t* __restrict__
   put(0);
   gload(min(1, nsteps - 1));
   __syncthreads();
+  auto infinite = [&]() __attribute__((always_inline)) {
+    return (uint32_t)__builtin_amdgcn_readfirstlane(
+        (int)__hip_atomic_load(&sinf, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+  };
   int s = 0;
   const int nfull = NB / SB;
 #pragma unroll 1
-  for (; s < nfull && !__builtin_amdgcn_readfirstlane(sinf); ++s) {
+  for (; s < nfull && !(infinite() >> (s & 1) & 1); ++s) {
     const int buf = s & 1;
     put(buf ^ 1);
     gload(min(s + 2, nsteps - 1));

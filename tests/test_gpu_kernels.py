@@ -148,6 +148,30 @@ def test_q8_gemm_step_edges(native, orc, monkeypatch, rows, k, tokens, nf):
     assert np.array_equal(_bits(y.download(np.float32, rows * tokens).reshape(tokens, rows)), _bits(want))
 
 
+@pytest.mark.parametrize("nf", ["1", "2"])
+@pytest.mark.parametrize("block", [0, 7, 8, 20, 31, 32, 33])
+def test_q8_gemm_infinite_scale_at_each_step(native, orc, monkeypatch, nf, block):
+    """Both tilings where the first infinite weight scale of a workgroup lies in its first, a middle,
+    the last whole and the partial last staging step (34 blocks in steps of 4 and 8): the fold goes
+    over to the plain form in that step, for that workgroup alone, and every value is the CPU fold's."""
+    monkeypatch.setenv("CAMELID_HIP_GEMM_NF", nf)
+    rows, k, tokens = 192, 34 * 32, 70
+    rng = np.random.default_rng(block)
+    wire = orc.quantize_q8_0_wire(rng.normal(0, 0.02, rows * k).astype(np.float32))
+    blocks = wire.reshape(rows, k // 32, 34)
+    for row, scale in ((3, 0x7C00), (40, 0xFC00), (130, 0x7C00)):
+        blocks[row, block, :2] = (scale & 0xFF, scale >> 8)
+    q, d = _repack(native, wire, rows, k)
+    pairs = [orc.quantize_q8_0(rng.normal(0, 1 + t % 5, k).astype(np.float32)) for t in range(tokens)]
+    xs, xq = np.stack([p[0] for p in pairs]), np.stack([p[1] for p in pairs])
+    wq, wd, dxq, dxs, y = _dev(q), _dev(d), _dev(xq), _dev(xs), _buf(rows * tokens * 4)
+    _ok(native.camelid_hip_q8_0_gemm(wq.ptr, wd.ptr, rows, k, dxq.ptr, dxs.ptr, tokens, y.ptr, None, None))
+    got = y.download(np.float32, rows * tokens).reshape(tokens, rows)
+    want = np.stack([orc.q8_0_gemv(wire, rows, k, xs[t], xq[t]) for t in range(tokens)])
+    assert np.isinf(want).any()
+    assert ((_bits(got) == _bits(want)) | (np.isnan(got) & np.isnan(want))).all()
+
+
 @pytest.mark.parametrize("rows,k,tokens,shift", [(4, 512, 1, 0), (16, 512, 8, 0), (20, 1024, 2, 0), (36, 8192, 5, 0),
                                                  (20, 8704, 7, 0), (16, 14336, 8, 0), (20, 1024, 3, 2), (20, 1024, 3, 1)])
 def test_q8_gemm_few_tokens(native, orc, rows, k, tokens, shift):
