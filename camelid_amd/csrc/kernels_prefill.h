@@ -246,6 +246,10 @@ __global__ __launch_bounds__(GMM_WAVES * 64) void k_gemv_mm(const int8_t* __rest
       for (int c = 0; c < 8; ++c) xv[c] = *reinterpret_cast<const v4i_t*>(xp + 64 * c);
     }
     if (lane < 32) sl[(lane & 3) * GMM_MAX + (lane >> 2)] = sc;
+    // (this wave's own LDS, read by all its lanes: wave-level ordering only)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
   auto w_at = [&](int tile, int sg) __attribute__((always_inline)) {
     return wq + (size_t)min(tile * GMM_ROWS + n, rows - 1) * K + sg * GMM_SEG + 16 * g;
