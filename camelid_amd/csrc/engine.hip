@@ -1381,22 +1381,72 @@ uint32_t q6m_tokens(uint32_t K) {
   return t;
 }
 
-constexpr uint32_t Q4K_MM_MIN = 1, Q6K_MM_MIN = 1;
+// Tokens per launch of the multi-token Q4_K GEMV at width K, at most T (its activations and terms
+// within 64 KB of LDS).
+uint32_t q4m_tokens(uint32_t K, uint32_t T) {
+  while (T > 1 && cm::gemv_q4k_multi_lds_bytes((int)K, (int)T) > 65536) --T;
+  return T;
+}
+
+// Whether the few-token kernels on the matrix cores (cm::k_gemv_q4k_mm, cm::k_gemv_q6k_mm) are
+// faster for T tokens than the multi-token GEMVs (cm::k_gemv_q4k_multi, cm::k_gemv_q6k_multi), by
+// estimates of both in us.  A matrix-core workgroup walks all of K for 16 rows whatever T is: a
+// start, a step per slice of 16 superblocks and round of resident workgroups, and more where a CU
+// has two of them.  A GEMV's time grows with T by the VALU work of its rows, or by the chain of one
+// row where rows are few; the activations in LDS limit its workgroups per CU, which costs a last
+// round that is partly empty and, at one or two per CU, their latency, and from 64 KB on further
+// launches.  The constants are a fit to 30 shapes of 256 to 151936 rows and 2048 to 16384 values
+// at 1 to 8 tokens, where no choice takes more than 1.05 of the GEMV's time, and on average 1.001
+// (Q4_K) and 1.005 (Q6_K) of the better kernel's.  Measured, GEMV / matrix cores:
+//   Q4_K [5120 x 4096]    1 token 5.8 / 11.3    4 8.5 / 11.4    6 12.3 / 11.6    8 15.3 / 11.9
+//        [4096 x 4096]    2       6.1 / 7.6     4 7.7 / 7.7     5 8.5 / 7.8      8 13.9 / 8.2
+//        [24576 x 4096]   1      15.3 / 20.8    2 18.7 / 20.8   3 21.5 / 20.7    8 59.3 / 21.1
+//        [4096 x 12288]   1      10.8 / 15.9    2 13.2 / 16.1   3 19.2 / 16.2    8 50.2 / 16.9
+//        [13824 x 5120]   1      13.7 / 32.1    4 23.8 / 32.9   6 38.0 / 33.4    8 56.7 / 34.0
+//   Q6_K [1024 x 4096]    1       4.0 / 7.1     4 6.1 / 7.9     6 7.4 / 8.3      7 8.1 / 7.7
+//        [4096 x 12288]   1      13.2 / 17.9    2 17.4 / 18.2   3 26.1 / 19.5    8 68.8 / 22.6
+//        [151936 x 4096]  1       123 / 107     2 163 / 116                      8 452 / 166
+// CAMELID_HIP_KQ_MM=0 / 1 forces the GEMVs / the matrix cores.
+bool kgemm_few_mm(const KMat& m, uint32_t T) {
+  if (const char* f = std::getenv("CAMELID_HIP_KQ_MM")) return std::atoi(f) != 0;
+  const int rows = (int)m.rows, K = (int)m.k;
+  auto cdiv = [](int a, int b) { return (a + b - 1) / b; };
+  const double k = 1e-3 * K, mvals = 1e-6 * rows * K;
+  if (m.quant == CAMELID_Q4_K) {
+    const int tiles = cdiv(rows, cm::Q4X_ROWS), slices = cdiv(K / 256, 2 * cm::Q4X_W);
+    const bool two = tiles > 256;  // workgroups on some CU
+    const double mm = 2.3 + cdiv(tiles, cm::Q4X_RESIDENT) * slices * (4.4 + (two && slices > 1 ? 3.1 : 0.0)) +
+                      (two && slices == 1 ? 5.2 : 0.0);
+    double multi = 0.0;
+    const uint32_t tt = q4m_tokens(m.k, T);
+    for (uint32_t t0 = 0; t0 < T; t0 += tt) {  // its launches
+      const int n = (int)std::min(tt, T - t0);
+      const int res = std::min(8, GFX950_LDS_PER_WORKGROUP / ((int)cm::gemv_q4k_multi_lds_bytes(K, n) + 1024));
+      const int per_cu = cdiv(rows, 4 * 256), rounds = cdiv(per_cu, res);
+      const double empty = rounds > 1 ? (double)rounds * res / per_cu : 1.0;
+      multi += 3.3 + 0.045 * mvals + n * std::max(0.103 * k, 0.051 * mvals) * empty * (res <= 2 ? 1.7 : 1.0);
+    }
+    return mm < multi;
+  }
+  if (T * m.k >= 28000) return true;
+  const int steps = cdiv(cdiv(rows, cm::Q6X_ROWS), cm::Q6X_CUS) * cdiv(K / 256, cm::Q6X_W);
+  return 5.4 + steps * (2.6 + 0.21 * T) < 2.8 + 0.36 * T + 1e-3 * rows * cdiv(K, 4096) * (0.44 + 0.28 * T);
+}
 
 // A K-quant projection over T tokens with Q8_K activation rows (kd [T][k/256], kq [T][k]):
-// y[t * ldy + row] (+ resid, same stride).  Q4_K: the matrix-core GEMM; Q6_K: for more than
-// Q6M_MAX tokens the class-major GEMM (needs m.w2 and xt, cm::q6g_act_bytes(T, k) bytes for
-// the class-major copy of kq) or else the sparse-MFMA GEMM, for fewer the multi-token GEMV.
+// y[t * ldy + row] (+ resid, same stride).  Up to Q4M_MAX = Q6M_MAX tokens: the few-token kernel on
+// the matrix cores or the multi-token GEMV (kgemm_few_mm).  More: Q4_K the matrix-core GEMM, Q6_K the
+// class-major GEMM (needs m.w2 and xt, cm::q6g_act_bytes(T, k) bytes for the class-major copy of
+// kq) or else the sparse-MFMA GEMM.
 void launch_kgemm(const KMat& m, uint32_t T, const float* kd, const int8_t* kq, float* y, uint32_t ldy,
                   const float* resid, hipStream_t s, int8_t* xt) {
-  if (m.quant == CAMELID_Q4_K && T >= Q4K_MM_MIN && T <= (uint32_t)cm::Q4X_MAX) {  // a few tokens, the matrix cores
+  if (m.quant == CAMELID_Q4_K && T <= (uint32_t)cm::Q4X_MAX && kgemm_few_mm(m, T)) {
     CM_LAUNCH(cm::k_gemv_q4k_mm, dim3(cm::q4x_grid((int)m.rows)), dim3(cm::Q4X_W * 64), cm::Q4X_LDS, s, m.a, m.b,
               (int)m.rows, (int)m.k, kd, kq, (int)T, y, (int)ldy, resid);
     return;
   }
   if (m.quant == CAMELID_Q4_K && T <= (uint32_t)cm::Q4M_MAX) {  // a few tokens (verify)
-    uint32_t tt = T;
-    while (tt > 1 && cm::gemv_q4k_multi_lds_bytes((int)m.k, (int)tt) > 65536) --tt;
+    const uint32_t tt = q4m_tokens(m.k, T);
     const uint32_t nsb = m.k / 256, it = (m.k / 32 + 63) / 64;
     for (uint32_t t0 = 0; t0 < T; t0 += tt) {
       const uint32_t n = std::min(tt, T - t0);
@@ -1435,7 +1485,7 @@ void launch_kgemm(const KMat& m, uint32_t T, const float* kd, const int8_t* kq, 
               dim3(cm::G6_NT), 0, s, m.a, m.b, m.sc, m.d, (int)m.rows, (int)m.k, kd, kq, (int)T, y, (int)ldy, resid);
     return;
   }
-  if (T >= Q6K_MM_MIN) {  // the matrix cores
+  if (kgemm_few_mm(m, T)) {
     const dim3 grid(cm::q6x_grid((int)m.rows)), block(cm::Q6X_W * 64);
     switch ((T + 1) / 2) {
 #define CM_Q6X(NP)                                                                                              \
@@ -1549,8 +1599,8 @@ float* pf_scratch(const camelid_hip_engine* e, uint32_t T, uint32_t pos0) {
 // One chunk of T prompt tokens at positions pos0.. through every layer; the residual rows
 // are in e->pf_h, the RoPE rows of the chunk at cosv / sinv.
 // A layer with K-quant projections over the chunk (the order of run_layer_generic per token):
-// RMSNorm rows to Q8_0 and Q8_K, each projection in its own format (Q4_K: k_gemm_q4k, Q6_K:
-// k_gemv_q6k_multi, Q8_0: launch_gemm), the attention rows also in f32 for a K-quant O.
+// RMSNorm rows to Q8_0 and Q8_K, each projection in its own format (K-quants: launch_kgemm, Q8_0:
+// launch_gemm), the attention rows also in f32 for a K-quant O.
 void prefill_layer_generic(camelid_hip_engine* e, uint32_t l, const float* cosv, const float* sinv, uint32_t T,
                            uint32_t pos0, float scale) {
   const camelid_hip_dims& d = e->d;

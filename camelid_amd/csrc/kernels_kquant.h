@@ -1053,6 +1053,10 @@ __global__ __launch_bounds__(KQ_NT) void k_gemv_q6k_multi(const uint8_t* __restr
 // meanwhile; the terms (d * y.d) * aux go to LDS, where one thread per (row, token, class) adds
 // them in superblock order; eight lanes then meet for the left fold from -0.0.  Rows of more than
 // Q6X_W superblocks go in slices, the class sums carried along.
+// Bound by the chain of one tile (load, 32 matrix instructions a token pair, the fold of 16 terms)
+// on small matrices, by the VALU work of forming the operands and HBM on large ones.  Measured
+// (us, k_gemv_q6k_multi / this): [4096 x 12288] 4 tokens 38.8 / 19.5, 8 tokens 68.8 / 22.6;
+// [1024 x 4096] 4 tokens 6.1 / 7.9; [151936 x 4096] 1 token 123 / 107, 8 tokens 452 / 166 (3.1 TB/s).
 // K % 256 == 0.  Dynamic LDS: q6x_lds_bytes(NP).
 constexpr int Q6X_W = 16;  // waves of a workgroup = superblocks of a slice
 constexpr int Q6X_ROWS = 16;
@@ -1708,6 +1712,10 @@ __global__ __launch_bounds__(KQ_NT) void k_gemv_q4k_multi(const uint8_t* __restr
 // meanwhile; terms through LDS, one thread per (row, token) folds them in superblock order; rows
 // of more than 2 Q4X_W superblocks in slices.  k_gemv_q4k_multi's VALU work is per token, this
 // one's is not.
+// Bound by the chain of one tile (load, 24 matrix instructions, the fold of 16 superblocks) on small
+// matrices, by HBM on large ones.  Measured (us, k_gemv_q4k_multi / this): [4096 x 4096] 4 tokens
+// 7.7 / 7.7, 8 tokens 13.9 / 8.2; [24576 x 4096] 4 tokens 25.9 / 20.8, 8 tokens 59.4 / 21.1;
+// [151936 x 4096] 8 tokens 334 / 79.5 (4.4 TB/s); [5120 x 4096] 4 tokens 8.5 / 11.4.
 // K % 256 == 0.  Dynamic LDS: Q4X_LDS.
 constexpr int Q4X_MAX = 8;
 constexpr int Q4X_W = 8;  // waves

@@ -762,15 +762,21 @@ def test_kquant_gemm_bit_exact(native, orc, quant, rows, k, T, ldy):
             assert np.array_equal(_bits(want), _bits(orc.kquant_gemv(quant, wire, rows, k, ydh[t], yqh[t])))
 
 
+@pytest.mark.parametrize("mm", ["0", "1"])
 @pytest.mark.parametrize("quant,rows,k,T", [(1, 3, 256, 4), (1, 16, 768, 8), (1, 17, 4096, 5), (1, 31, 4352, 7),
                                             (1, 8209, 512, 6), (1, 20, 16384, 8), (2, 3, 256, 4), (2, 16, 3840, 8),
                                             (2, 17, 4096, 5), (2, 31, 4352, 7), (2, 4113, 512, 6), (2, 20, 16384, 8),
-                                            (1, 40, 8448, 2), (2, 40, 8448, 2), (1, 33, 2048, 3), (2, 33, 2048, 3)])
-def test_kquant_few_tokens_edges(native, orc, quant, rows, k, T):
-    """The few-token kernels at their edges: one superblock, an odd number of them, a slice and one
-    superblock more, several slices; rows short of, at and past a 16-row tile and more tiles than
-    resident workgroups; odd token counts; scales and quants over their whole ranges (Q6_K: scale
-    products of +4096 and -4064 in rows 0 and 1).  Every value is the CPU dot's, bit for bit."""
+                                            (1, 40, 8448, 2), (2, 40, 8448, 2), (1, 33, 2048, 3), (2, 33, 2048, 3),
+                                            (1, 3, 256, 1), (2, 3, 256, 1), (2, 35, 4352, 1), (1, 8209, 4352, 3),
+                                            (2, 4113, 4352, 5)])
+def test_kquant_few_tokens_edges(native, orc, monkeypatch, quant, rows, k, T, mm):
+    """The few-token kernels at their edges, the matrix-core ones and the multi-token GEMVs forced in
+    turn: one superblock, an odd number of them, a slice and one superblock more, several slices;
+    rows short of, at and past a 16-row tile and more tiles than resident workgroups, with one slice
+    and with a short second one; one token and odd token counts; scales and quants over their whole
+    ranges (Q6_K: scale products of +4096 and -4064 in rows 0 and 1).  Every value is the CPU dot's,
+    bit for bit."""
+    monkeypatch.setenv("CAMELID_HIP_KQ_MM", mm)
     rng = np.random.default_rng(rows + 3 * k + T + quant)
     wire = _kquant_wire(orc, rng, quant, rows, k)
     if quant == 2:
