@@ -1527,9 +1527,8 @@ void launch_gemm(const Q8Mat& m, uint32_t T, const int8_t* xq, const float* xs, 
         break;
     }
   }
-  // a few tokens: weights streamed once by GEMV-shaped workgroups (16-byte loads of the scales too)
-  if (T <= (uint32_t)cm::GMM_MAX && m.k % cm::GMM_SEG == 0 &&
-      ((reinterpret_cast<uintptr_t>(m.d) | reinterpret_cast<uintptr_t>(xs)) & 15) == 0) {
+  // a few tokens: weights streamed once by GEMV-shaped workgroups
+  if (T <= (uint32_t)cm::GMM_MAX && m.k % cm::GMM_SEG == 0) {
     const dim3 grid(cm::gemv_mm_grid((int)m.rows, (int)m.k)), block(64 * cm::gemv_mm_waves((int)m.k));
     const size_t lds = cm::gemv_mm_lds_bytes((int)m.k);
     if (cm::gemv_mm_sliced((int)m.k))

@@ -194,11 +194,14 @@ __global__ __launch_bounds__(256) void k_gemv_multi(const int8_t* __restrict__ w
 // 10.1 / 8.6, [3072 x 3072] 7.8 / 5.9, [3072 x 8192] 24.9 / 11.4, [128256 x 3072] 165 / 82 (5.1
 // TB/s), [28672 x 4096] 58.8 / 31.8; 4 tokens: [16384 x 3072] 15.0 / 14.3, [3072 x 3072] 6.1 / 5.8;
 // 3 tokens: 13.6 / 14.3, [5120 x 3072] 7.0 / 8.2, [28672 x 4096] 25.6 / 30.7, [128256 x 3072] 77.6 / 77.8.
-// K % GMM_SEG == 0; scales of either side 16-byte aligned.
+// K % GMM_SEG == 0; scales of either side at any alignment of their type (16-byte loads all the same:
+// global memory takes them at any byte).
 constexpr int GMM_MAX = 8;
 constexpr int GMM_SEG = 512;   // values of K per wave and slice: 8 chunks of two blocks
 constexpr int GMM_WAVES = 16;  // waves of a workgroup at most
 constexpr int GMM_ROWS = 16;
+typedef uint32_t gmm_u4_t __attribute__((ext_vector_type(4), aligned(2)));  // eight f16 scales
+typedef float gmm_f4_t __attribute__((ext_vector_type(4), aligned(4)));     // four f32 scales
 // waves per workgroup (the last one idle in the products at K = 512: the fold wants two)
 inline int gemv_mm_waves(int K) {
   const int segs = K / GMM_SEG, slices = (segs + GMM_WAVES - 1) / GMM_WAVES;
@@ -232,20 +235,21 @@ __global__ __launch_bounds__(GMM_WAVES * 64) void k_gemv_mm(const int8_t* __rest
   const int xt = 2 * (n >> 2) + (n & 1);
   const bool xon = xt < T && (g >> 1) == ((n >> 1) & 1);
   int4 wv[8];
-  uint4 dv[2];
+  gmm_u4_t dv[2];
   v4i_t xv[8];
   float4* sl = terms + (size_t)W * 8 * 64 + wave * (GMM_MAX * GMM_SEG / 32 / 4);
   auto load_x = [&](int sg) __attribute__((always_inline)) {
     const int8_t* xp = xq + (size_t)min(xt, T - 1) * K + sg * GMM_SEG + 16 * g;
     // (lane: token lane / 4 % 8, blocks 4 (lane % 4) .. + 3)
-    const float4 sc = reinterpret_cast<const float4*>(xs + (size_t)min((lane >> 2) & 7, T - 1) * NB + sg * 16)[lane & 3];
+    const gmm_f4_t sc =
+        reinterpret_cast<const gmm_f4_t*>(xs + (size_t)min((lane >> 2) & 7, T - 1) * NB + sg * 16)[lane & 3];
 #pragma unroll
     for (int c = 0; c < 8; ++c) xv[c] = v4i_t{0, 0, 0, 0};
     if (xon) {
 #pragma unroll
       for (int c = 0; c < 8; ++c) xv[c] = *reinterpret_cast<const v4i_t*>(xp + 64 * c);
     }
-    if (lane < 32) sl[(lane & 3) * GMM_MAX + (lane >> 2)] = sc;
+    if (lane < 32) sl[(lane & 3) * GMM_MAX + (lane >> 2)] = make_float4(sc.x, sc.y, sc.z, sc.w);
     // (this wave's own LDS, read by all its lanes: wave-level ordering only)
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -255,9 +259,9 @@ __global__ __launch_bounds__(GMM_WAVES * 64) void k_gemv_mm(const int8_t* __rest
     return wq + (size_t)min(tile * GMM_ROWS + n, rows - 1) * K + sg * GMM_SEG + 16 * g;
   };
   auto d_at = [&](int tile, int sg) __attribute__((always_inline)) {
-    return reinterpret_cast<const uint4*>(wd + (size_t)min(tile * GMM_ROWS + n, rows - 1) * NB + sg * 16);
+    return reinterpret_cast<const gmm_u4_t*>(wd + (size_t)min(tile * GMM_ROWS + n, rows - 1) * NB + sg * 16);
   };
-  auto load_w = [&](const int8_t* wn, const uint4* dn) __attribute__((always_inline)) {
+  auto load_w = [&](const int8_t* wn, const gmm_u4_t* dn) __attribute__((always_inline)) {
 #pragma unroll
     for (int c = 0; c < 8; ++c) wv[c] = *reinterpret_cast<const int4*>(wn + 64 * c);
 #pragma unroll
@@ -265,7 +269,7 @@ __global__ __launch_bounds__(GMM_WAVES * 64) void k_gemv_mm(const int8_t* __rest
   };
   // the terms of a segment; with next, a chunk's registers take the next segment's loads as soon
   // as its product is issued
-  auto segment = [&](auto nextc, const int8_t* wn, const uint4* dn) __attribute__((always_inline)) {
+  auto segment = [&](auto nextc, const int8_t* wn, const gmm_u4_t* dn) __attribute__((always_inline)) {
     constexpr bool next = decltype(nextc)::value;
     float4* tp = terms + (size_t)wave * 8 * 64 + lane;
 #pragma unroll
@@ -295,7 +299,7 @@ __global__ __launch_bounds__(GMM_WAVES * 64) void k_gemv_mm(const int8_t* __rest
   };
   int tile = blockIdx.x, s0 = 0;
   const int8_t* wn = w_at(tile, min(wave, segs - 1));
-  const uint4* dn = d_at(tile, min(wave, segs - 1));
+  const gmm_u4_t* dn = d_at(tile, min(wave, segs - 1));
   if (wave < segs) {
     load_w(wn, dn);
     load_x(wave);

@@ -173,11 +173,12 @@ def test_q8_gemm_infinite_scale_at_each_step(native, orc, monkeypatch, nf, block
 
 
 @pytest.mark.parametrize("rows,k,tokens,shift", [(4, 512, 1, 0), (16, 512, 8, 0), (20, 1024, 2, 0), (36, 8192, 5, 0),
-                                                 (20, 8704, 7, 0), (16, 14336, 8, 0), (20, 1024, 3, 2), (20, 1024, 3, 1)])
+                                                 (20, 8704, 7, 0), (16, 14336, 8, 0), (20, 1024, 3, 2), (20, 1024, 3, 1),
+                                                 (36, 2048, 4, 1), (36, 2048, 8, 1), (100, 4096, 5, 3), (36, 8704, 6, 1)])
 def test_q8_gemm_few_tokens(native, orc, rows, k, tokens, shift):
     """The few-token kernel at its edges: one segment (a wave without products), the most segments of
     one slice, two slices (9 + 8 and 14 + 14), rows past a 16-row tile, odd token counts; and scales
-    at a 2-byte (shift 1) or 4-byte (2) offset, which it does not take."""
+    at a 2-byte (shift 1) or 4-byte (2) offset, where its 16-byte loads of them are misaligned."""
     rng = np.random.default_rng(rows + 3 * k + tokens)
     wire = orc.quantize_q8_0_wire(rng.normal(0, 0.02, rows * k).astype(np.float32))
     q, d = _repack(native, wire, rows, k)
