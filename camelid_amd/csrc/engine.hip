@@ -1507,13 +1507,30 @@ void launch_kgemm(const KMat& m, uint32_t T, const float* kd, const int8_t* kq, 
   }
 }
 
+// Whether cm::k_gemv_mm (16 rows per workgroup, matrix cores) is faster for T tokens than
+// cm::k_gemv_multi (4 rows, VALU) at a width the latter has.  The GEMV's time grows with T by its
+// VALU work, k_gemv_mm's does not: the GEMV up to 3 tokens, k_gemv_mm from 5 on (at worst 1.04,
+// [5120 x 4096] x 5).  At 4 tokens k_gemv_mm loses where its workgroups do not fill the device:
+// long rows in fewer than 128 tiles, 257 to 383 tiles of short rows (some CUs have a second one),
+// and 4096 values above 256 tiles, where the GEMV's four pieces per lane and token come out even.
+// Measured at 4 tokens, GEMV / k_gemv_mm (us): [1024 x 8192] 8.9 / 9.7, [4096 x 8192] 14.1 / 11.7,
+// [5120 x 2048] 5.8 / 6.4, [32000 x 2048] 18.5 / 15.0, [5120 x 3072] 7.7 / 7.8, [16384 x 3072]
+// 14.8 / 12.9, [4096 x 4096] 8.6 / 8.4, [6144 x 4096] 10.2 / 11.1, [28672 x 4096] 27.9 / 30.7.
+bool gemv_mm_faster(uint32_t rows, uint32_t k, uint32_t T) {
+  if (T != 4) return T > 4;
+  const uint32_t tiles = (rows + cm::GMM_ROWS - 1) / cm::GMM_ROWS;
+  if (tiles < 128) return k < 4096;
+  if (k == 4096) return tiles <= 256;
+  return k > 4096 || tiles <= 256 || tiles >= 384;
+}
+
 // 64 x 64 tiles from this many of them on (256 CUs), else 32 x 32 ones.  Measured (us, 64 / 32):
 // [3072 x 3072] 200 tokens (192 tiles of 64) 26.3 / 20.1, 300 (240) 26.2 / 24.6, 511 (384) 31.5 /
 // 34.3; [11264 x 2048] 37 tokens (176) 18.2 / 13.9, 127 (352) 22.7 / 24.7.
 constexpr int GEMM_BIG_TILES = 288;
 void launch_gemm(const Q8Mat& m, uint32_t T, const int8_t* xq, const float* xs, float* y, const float* resid,
                  hipStream_t s) {
-  if (T <= (uint32_t)cm::GMT_MAX && m.k <= 8192) {  // up to three tokens
+  if (T <= (uint32_t)cm::GMT_MAX && m.k <= 8192 && !gemv_mm_faster(m.rows, m.k, T)) {
     const uint32_t grid = (m.rows + cm::GMT_ROWS - 1) / cm::GMT_ROWS;
     const size_t lds = cm::gemv_multi_lds_bytes((int)m.k, (int)T);
     switch (m.k) {

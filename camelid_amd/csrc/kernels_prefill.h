@@ -66,12 +66,12 @@ __global__ __launch_bounds__(64) void k_argmax_rows_finish(const float* __restri
 
 // ---------------------------------------------------------------------------
 // Y[t] = W . X[t] (+ resid[t]) for 1 <= T <= GMT_MAX tokens (the shortest verify and
-// prefill chunks; k_gemv_mm from four on): the single-token GEMV's arithmetic for every (row, token) -- exact int32
+// prefill chunks; k_gemv_mm above, and at four where it is faster): the single-token GEMV's arithmetic for every (row, token) -- exact int32
 // block dots, terms ((float)dot * d_w) * d_x, the in-order fold over blocks -- with each
 // weight chunk loaded once and dotted with all T activations (a 64-token matrix-core tile
 // would leave most CUs idle at this size).  4 waves x GMT_RPW rows per workgroup.
 // Dynamic LDS: gemv_multi_lds_bytes(K, T).
-constexpr int GMT_MAX = 3;
+constexpr int GMT_MAX = 4;
 constexpr int GMT_RPW = 1;
 constexpr int GMT_ROWS = 4 * GMT_RPW;
 // LDS: the activations [T][K] i8 and their scales [T][K/32] f32, each rounded up to whole
@@ -190,10 +190,10 @@ __global__ __launch_bounds__(256) void k_gemv_multi(const int8_t* __restrict__ w
 // tile's weights are on their way while this one's terms are formed and added.  More than
 // GMM_WAVES segments go in slices with the sums carried along.
 // Bound by HBM on large matrices, by the latency of one load, product and fold on small ones.
-// Measured, 8 tokens (us, k_gemv_multi / this): [16384 x 3072] 26.1 / 14.9, [5120 x 3072]
-// 10.1 / 8.6, [3072 x 3072] 7.8 / 5.9, [3072 x 8192] 24.9 / 11.4, [128256 x 3072] 165 / 82 (5.1
-// TB/s), [28672 x 4096] 58.8 / 31.8; 4 tokens: [16384 x 3072] 15.0 / 14.3, [3072 x 3072] 6.1 / 5.8;
-// 3 tokens: 13.6 / 14.3, [5120 x 3072] 7.0 / 8.2, [28672 x 4096] 25.6 / 30.7, [128256 x 3072] 77.6 / 77.8.
+// Measured, weights from HBM, 8 tokens (us, k_gemv_multi / this): [16384 x 3072] 24.4 / 13.4, [5120 x
+// 3072] 10.2 / 8.0, [3072 x 3072] 7.9 / 5.6, [3072 x 8192] 25.1 / 10.8, [128256 x 3072] 156 / 80 (5.2
+// TB/s), [28672 x 4096] 55.6 / 31.6; two slices (the prefill GEMM / this): [4096 x 14336] 44.6 / 19.7,
+// [5120 x 13824] 52 / 32.3.
 // K % GMM_SEG == 0; scales of either side at any alignment of their type (16-byte loads all the same:
 // global memory takes them at any byte).
 constexpr int GMM_MAX = 8;

@@ -192,6 +192,22 @@ def test_q8_gemm_few_tokens(native, orc, rows, k, tokens, shift):
     assert np.array_equal(_bits(y.download(np.float32, rows * tokens).reshape(tokens, rows)), _bits(want))
 
 
+@pytest.mark.parametrize("rows,k", [(36, 2048), (2048, 4096), (4096, 4096), (4112, 4096), (5120, 3072), (8192, 2048),
+                                    (1024, 8192), (2048, 5632)])
+def test_q8_gemm_four_tokens(native, orc, rows, k):
+    """Four tokens on both sides of the lines between the multi-token GEMV and the matrix cores."""
+    rng = np.random.default_rng(rows + k)
+    wire = orc.quantize_q8_0_wire(rng.normal(0, 0.02, rows * k).astype(np.float32))
+    q, d = _repack(native, wire, rows, k)
+    pairs = [orc.quantize_q8_0(rng.normal(0, 1 + t % 5, k).astype(np.float32)) for t in range(4)]
+    xs, xq = np.stack([p[0] for p in pairs]), np.stack([p[1] for p in pairs])
+    resid = rng.normal(0, 1, (4, rows)).astype(np.float32)
+    wq, wd, dxq, dxs, y = _dev(q), _dev(d), _dev(xq), _dev(xs), _dev(resid)
+    _ok(native.camelid_hip_q8_0_gemm(wq.ptr, wd.ptr, rows, k, dxq.ptr, dxs.ptr, 4, y.ptr, y.ptr, None))
+    want = resid + np.stack([orc.q8_0_gemv(wire, rows, k, xs[t], xq[t]) for t in range(4)])
+    assert np.array_equal(_bits(y.download(np.float32, rows * 4).reshape(4, rows)), _bits(want))
+
+
 @pytest.mark.parametrize("rows,k,tokens", [(4112, 8704, 5), (5120, 13824, 8), (8192, 9728, 1), (5120, 17408, 4)])
 def test_q8_gemm_few_tokens_short_last_slice(native, orc, rows, k, tokens):
     """The few-token kernel where a row's K goes in two or three slices, the last one short, and a
