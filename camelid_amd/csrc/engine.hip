@@ -1569,16 +1569,26 @@ void launch_gemm(const Q8Mat& m, uint32_t T, const int8_t* xq, const float* xs, 
 }
 
 // Whether the tiled attention of a prefill chunk (cm::k_attn_prefill_mm: 16 rows of a KV head per
-// workgroup) is faster than one workgroup per (head, token) (cm::k_attn_prefill).  The per-token
-// kernel does about 32,000 (head, token, position) terms of 128 dims per us over the whole device;
-// a tile's time is its own latency, about 6 us + 0.072 us per position, as long as the device
-// holds all tiles at once, and about half the per-token kernel's time per term beyond.  Measured
-// (us, per token / tiled): 24 heads of 128 dims, 511 tokens 96 / 62, 32 tokens at 2000 positions
-// 54 / 147, 16 at 300 12 / 31; 32 heads of 64 dims, 127 tokens 12 / 17.
-bool attn_prefill_tiled(uint32_t hd, uint32_t n_heads, uint32_t T, uint32_t pos0) {
+// workgroup) is faster than one workgroup per (head, token) (cm::k_attn_prefill), by estimates of
+// both in us.  Per token: the (head, token, position) terms, in units of 128 dims and with 40
+// positions for a workgroup's own cost, at 36,000 per us over the device, or in proportion to the
+// workgroups that fit a CU beside their scores in LDS (4 bytes per position: 12,000 positions leave
+// three).  Tiled: a tile's own latency, 6 us + 0.07 us per position, or its share of the issue slots
+// where a CU has several tiles, at the chunk's mean position.  Fitted to 396 shapes (16 to 32 heads
+// of 64 and 128 dims, 8 to 511 tokens at positions 0 to 15800): 1.002 of the better kernel's time on
+// average, 1.12 at worst.  Measured (us, per token / tiled):
+//   32 heads, 8 KV, of 128: 511 tokens at 0 122 / 67, 128 at 0 18 / 17, 64 at 2048 107 / 142, 64 at
+//   12288 868 / 854, 64 at 15800 1420 / 1097, 192 at 4096 617 / 399;
+//   24 heads, 8 KV, of 128: 511 at 0 92 / 58, 32 at 2048 51 / 140, 96 at 15800 1683 / 1092;
+//   32 heads, 4 KV, of 64: 511 at 0 69 / 53, 192 at 512 58 / 71, 256 at 4096 436 / 466, 128 at
+//   15800 2456 / 1270.
+bool attn_prefill_tiled(uint32_t hd, uint32_t n_heads, uint32_t n_kv, uint32_t T, uint32_t pos0) {
   if (!cm::apm_hd_ok((int)hd)) return false;
-  const double pos = pos0 + 0.5 * T, terms = (double)T * n_heads * pos * hd / 128.0;
-  return terms > 32000.0 * (3.0 + 0.075 * ((double)pos0 + T));
+  const double end = (double)pos0 + T, mean = pos0 + 0.5 * T, terms = (double)T * n_heads * (mean + 40) * hd / 128.0;
+  const int fit = GFX950_LDS_PER_WORKGROUP / (4 * (int)(pos0 + T) + 512);
+  const double rate = std::min(36000.0, fit * (hd == 64 ? 6000.0 : 9500.0));
+  const double per_cu = n_kv * cm::apm_tiles((int)(n_heads / n_kv), (int)T) / 256.0;
+  return terms > rate * (6.0 + 0.07 * std::max(end, mean * (0.6 + 0.5 * per_cu)));
 }
 
 // Causal attention of a prefill chunk: tiled when scratch (cm::apm_scratch floats) is given, else
@@ -1609,7 +1619,9 @@ void launch_attn_prefill(uint32_t hd, uint32_t n_heads, uint32_t n_kv, uint32_t 
 
 // The scratch of a chunk that runs the tiled attention, else null.
 float* pf_scratch(const camelid_hip_engine* e, uint32_t T, uint32_t pos0) {
-  return pos0 + T >= e->att_tile_pos && attn_prefill_tiled(e->d.head_dim, e->d.n_heads, T, pos0) ? e->pf_sc : nullptr;
+  const camelid_hip_dims& d = e->d;
+  if (pos0 + T < e->att_tile_pos || !attn_prefill_tiled(d.head_dim, d.n_heads, d.n_kv_heads, T, pos0)) return nullptr;
+  return e->pf_sc;
 }
 
 // One chunk of T prompt tokens at positions pos0.. through every layer; the residual rows
@@ -2839,7 +2851,7 @@ int camelid_hip_attention_prefill(const float* qrot, const uint16_t* kc, const u
   // CAMELID_HIP_ATT_TILE: 1 the tiled kernel wherever it applies, 0 never, else by size; its score
   // scratch is allocated for the call
   const char* te = std::getenv("CAMELID_HIP_ATT_TILE");
-  const bool tiled = te ? std::atoi(te) != 0 && cm::apm_hd_ok((int)hd) : attn_prefill_tiled(hd, n_heads, tokens, pos0);
+  const bool tiled = te ? std::atoi(te) != 0 && cm::apm_hd_ok((int)hd) : attn_prefill_tiled(hd, n_heads, n_kv, tokens, pos0);
   float* scratch = nullptr;
   if (tiled && hipMalloc(&scratch, cm::apm_scratch((int)n_heads, (int)n_kv, (int)tokens, (size_t)pos0 + tokens) * 4) != hipSuccess)
     return fail(nullptr, "scratch allocation failed");

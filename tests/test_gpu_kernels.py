@@ -611,6 +611,33 @@ def test_attention_prefill_bit_exact(native, orc, monkeypatch, nh, nkv, hd, pos0
         assert np.array_equal(_bits(gxs[t]), _bits(ws)) and np.array_equal(gxq[t], wq)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,pos0,T", [(32, 8, 128, 15800, 64), (32, 4, 64, 12288, 128), (32, 4, 64, 512, 192),
+                                             (24, 8, 128, 0, 256), (24, 8, 128, 2048, 32), (16, 2, 128, 9001, 77)])
+def test_attention_prefill_by_size(native, orc, monkeypatch, nh, nkv, hd, pos0, T):
+    """Shapes on both sides of the line between the tiled and the per-token prefill attention, the
+    scores of the longest at the limit of two workgroups' LDS: the one that the size picks and
+    either forced give the same bits, f32 and Q8_0."""
+    rng = np.random.default_rng(nh + pos0 + T)
+    max_pos = (pos0 + T + 7) // 8 * 8
+    kd, vd = (rng.normal(0, s, nkv * max_pos * hd).astype(np.float16) for s in (1.5, 1))
+    q = rng.normal(0, 1, (T, nh * hd)).astype(np.float32)
+    scale = float(np.float32(1) / np.sqrt(np.float32(hd)))
+    dq, dk, dv = _dev(q), _dev(kd), _dev(vd)
+    got = []
+    for tile in (None, "0", "1"):
+        monkeypatch.delenv("CAMELID_HIP_ATT_TILE", raising=False)
+        if tile:
+            monkeypatch.setenv("CAMELID_HIP_ATT_TILE", tile)
+        out, xq, xs = _buf(T * nh * hd * 4), _buf(T * nh * hd), _buf(T * nh * hd // 32 * 4)
+        _ok(native.camelid_hip_attention_prefill(dq.ptr, dk.ptr, dv.ptr, 0, nh, nkv, hd, max_pos, pos0, T, scale,
+                                                 out.ptr, xq.ptr, xs.ptr, None))
+        got.append((out.download(np.uint32, T * nh * hd), xq.download(np.int8, T * nh * hd),
+                    xs.download(np.uint32, T * nh * hd // 32)))
+    assert np.isfinite(got[0][0].view(np.float32)).all()
+    for other in got[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(got[0], other))
+
+
 @pytest.mark.parametrize("nh,nkv,hd,pos0,T", [(5, 1, 128, 15, 7), (20, 1, 64, 31, 3), (3, 3, 64, 63, 18),
                                              (6, 2, 128, 0, 16), (16, 8, 128, 112, 33), (8, 1, 64, 47, 2)])
 def test_attention_prefill_tile_edges(native, orc, monkeypatch, nh, nkv, hd, pos0, T):
