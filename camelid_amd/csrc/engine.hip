@@ -1524,10 +1524,13 @@ bool gemv_mm_faster(uint32_t rows, uint32_t k, uint32_t T) {
   return k > 4096 || tiles <= 256 || tiles >= 384;
 }
 
-// 64 x 64 tiles from this many of them on (256 CUs), else 32 x 32 ones.  Measured (us, 64 / 32):
-// [3072 x 3072] 200 tokens (192 tiles of 64) 26.3 / 20.1, 300 (240) 26.2 / 24.6, 511 (384) 31.5 /
-// 34.3; [11264 x 2048] 37 tokens (176) 18.2 / 13.9, 127 (352) 22.7 / 24.7.
-constexpr int GEMM_BIG_TILES = 288;
+// 64 x 64 tiles from this many of them on (256 CUs), else 32 x 32 ones: a last round of big tiles
+// that fills few CUs costs more than the small tiles' extra operand reads.  Measured (us, 64 / 32):
+// [3072 x 3072] 300 tokens (240 tiles of 64) 26.2 / 23.2, 400 (336) 31.5 / 28.8, 511 (384) 32.0 /
+// 32.8; [4096 x 14336] 300 (320) 130 / 116, 400 (448) 131 / 153; [2560 x 2048] 511 (320) 22.3 /
+// 20.8; [5120 x 3072] 256 (320) 31.9 / 29.1, 300 (400) 31.9 / 36.7; [3072 x 8192] 400 (336) 75.0 /
+// 67.7, 511 (384) 75.6 / 78.9; [11264 x 2048] 100 (352) 23.1 / 23.3, 127 (352) 23.0 / 24.1.
+constexpr int GEMM_BIG_TILES = 352;
 void launch_gemm(const Q8Mat& m, uint32_t T, const int8_t* xq, const float* xs, float* y, const float* resid,
                  hipStream_t s) {
   if (T <= (uint32_t)cm::GMT_MAX && m.k <= 8192 && !gemv_mm_faster(m.rows, m.k, T)) {
