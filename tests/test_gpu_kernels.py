@@ -669,6 +669,56 @@ def test_attention_prefill_tile_edges(native, orc, monkeypatch, nh, nkv, hd, pos
         assert same.all(), f"token {t}"
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+def test_attention_prefill_subnormal_products(native, orc, monkeypatch, hd):
+    """Products below the normal range on either side of the prefill attention, both kernels.
+    Outputs: position 0 takes the softmax with V = 0 and the other exponentials are subnormal
+    (scores 89 to 102 below it), so every output is a sum of subnormal products: the oracle's bits,
+    nonzero.  Scores: q of 2^-126 and a scale of 2^126, so that every q k product is subnormal or just
+    above and the softmax shows it: the tiled kernel's bits are the per-token one's, and the outputs
+    near those of the same call with q and scale at ordinary sizes."""
+    nh, nkv, pos0, T = 4, 2, 21, 19
+    rng = np.random.default_rng(hd)
+    max_pos = (pos0 + T + 7) // 8 * 8
+
+    def run(q, kb, vb, scale):
+        kd, vd = _kv_device(kb, vb)
+        dq, dk, dv = _dev(q), _dev(kd), _dev(vd)
+        res = {}
+        for tile in ("0", "1"):
+            monkeypatch.setenv("CAMELID_HIP_ATT_TILE", tile)
+            out, xq, xs = _buf(T * nh * hd * 4), _buf(T * nh * hd), _buf(T * nh * hd // 32 * 4)
+            _ok(native.camelid_hip_attention_prefill(dq.ptr, dk.ptr, dv.ptr, 0, nh, nkv, hd, max_pos, pos0, T,
+                                                     float(np.float32(scale)), out.ptr, xq.ptr, xs.ptr, None))
+            res[tile] = out.download(np.float32, T * nh * hd).reshape(T, nh * hd)
+        assert np.array_equal(_bits(res["0"]), _bits(res["1"]))
+        return res["1"]
+
+    scale = np.float32(1) / np.sqrt(np.float32(hd))
+    kf = np.zeros((1, nkv, max_pos, hd), np.float32)
+    kf[..., 0] = rng.uniform(-9.75, -8.25, (1, nkv, max_pos))
+    kf[..., 0, 0] = 8.0
+    vf = rng.uniform(0.25, 2, (1, nkv, max_pos, hd)).astype(np.float32)
+    vf[:, :, 0] = 0.0
+    q = np.zeros((T, nh, hd), np.float32)
+    q[..., 0] = 5.55 / scale
+    q = q.reshape(T, nh * hd)
+    kb, vb = orc.f32_to_f16(kf), orc.f32_to_f16(vf)
+    got = run(q, kb, vb, scale)
+    kl, vl = orc.f16_to_f32(kb[0]).ravel(), orc.f16_to_f32(vb[0]).ravel()
+    want = np.stack([orc.attention(q[t], kl, vl, nh, nkv, hd, max_pos, pos0 + t + 1) for t in range(T)])
+    assert ((want > 0) & (want < np.finfo(np.float32).tiny)).all()
+    assert np.array_equal(_bits(got), _bits(want))
+
+    kb, vb = (orc.f32_to_f16(rng.normal(0, 1, (1, nkv, max_pos, hd)).astype(np.float32)) for _ in range(2))
+    q = rng.normal(0, 1, (T, nh * hd)).astype(np.float32)
+    tiny = run(q * np.float32(2.0**-126), kb, vb, scale * np.float32(2.0**126))
+    # q and each product lose at most 2^-150 to the subnormal grid, 2^-24 once scaled; with k up to
+    # 4 and scale at most 1/8 a score moves by hd (4 + 1) 2^-24 / 8, an output (v up to 4) by eight
+    # times that at most
+    np.testing.assert_allclose(tiny, run(q, kb, vb, scale), rtol=0, atol=hd * 2.0**-24 * 5)
+
+
 def test_quantize_q8_k_bit_exact(native, orc):
     """Q8_K activation quantizer == quantize_q8_k_blocks, incl. zero blocks, |max| ties (first
     wins), one-hot and huge/tiny blocks; per-32 sums of the quants."""
