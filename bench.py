@@ -35,8 +35,10 @@ INT8_PEAK_TOPS = 5000.0  # MI355X dense int8 matrix-core peak, AMD published
 HEADLINE = "llama-3.2-3b"
 ARCH = {"llama-3.2-3b": "Llama-3.2-3B-arch Q8_0", "tinyllama-1.1b": "TinyLlama-1.1B-arch Q8_0",
         "mistral-7b-v0.3": "Mistral-7B-v0.3-arch Q8_0 (8K context)", "qwen3-8b": "Qwen3-8B-arch Q4_K_M"}
-# MI355X peak engine clock (AMD published), for the VALU ceiling of the prefill GEMM's fold
-PEAK_CLOCK_HZ = 2.4e9
+# The Q8_0 prefill GEMM's fold (float(dot) * w_scale as one FMA, * x_scale, add) of 1024 outputs and
+# one block on one SIMD, operands in registers, measured with all SIMDs at it: the ceiling that the
+# block-ordered fold puts on the GEMM
+FOLD_NS_PER_1024 = 50.7
 # Measured HBM bytes per launch of the dominant kernel class, not measured by this script:
 # rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE passes over `bench.py --probe-traffic`, each
 # scaled by what the same counter reads for a device copy of known size, averaged over the
@@ -197,7 +199,8 @@ def run_sweep_kquant(tokens: int = 512, iters: int = 20) -> dict:
         us = ms.value / iters * 1e3
         ops = 2.0 * rows * k * T
         q6 = "k_gemm_q6k" if os.environ.get("CAMELID_HIP_Q6K_GEMM2") == "0" else "k_gemm_q6k2"
-        name = "k_gemm_q4k" if quant == 1 else (q6 if T > 8 else "k_gemv_q6k_multi")
+        few = "q4k" if quant == 1 else "q6k"  # up to 8 tokens: the size picks one of two kernels
+        name = f"k_gemv_{few}_mm or _multi" if T <= 8 else "k_gemm_q4k" if quant == 1 else q6
         out.append({"quant": "Q4_K" if quant == 1 else "Q6_K", "kernel": name, "shape": [rows, k], "tokens": T,
                     "us": round(us, 1), "tops": round(ops / us / 1e6, 1),
                     "mfma_frac": round(ops / us / 1e6 / INT8_PEAK_TOPS, 4)})
@@ -576,20 +579,15 @@ def main() -> int:
         g = pprof["prefill_gemm"]
         tops = g["bytes"] / (g["ms"] * 1e-3) / 1e12 if g["ms"] else 0.0
         # the bit-exact fold costs 3 unpacked VALU ops per output row, token and 32-wide block
-        # (64 int8 ops): float(dot) * w_scale as one mixed FMA on the dot offset by 1.5 * 2^23,
-        # the product with the activation scale, the add; a ceiling of 64 lanes x clock / 3 x 64
-        # ops per CU (the plain form's 4 ops, for matrices with an infinite weight scale, only
-        # lowers it)
-        fold_ceiling = n_cu * 64 * PEAK_CLOCK_HZ / 3 * 64 / 1e12
-        # (the same rate over the ceiling of the 4-operation fold -- convert, x w_scale, x x_scale,
-        # add -- which the GEMM used before the offset accumulator: the figure earlier builds reported)
-        fold4_ceiling = fold_ceiling * 3 / 4
+        # (64 int8 ops): float(dot) * w_scale as one FMA on the dot offset by 1.5 * 2^23, the product
+        # with the activation scale, the add (the plain form's 4 ops, for matrices with an infinite
+        # weight scale, only lowers the ceiling; K-quant projections fold differently)
+        fold_ceiling = n_cu * 4 * 1024 * 64 / (FOLD_NS_PER_1024 * 1e-9) / 1e12
         prefill_mm = {"tokens": P - 1, "gemm_tops": round(tops, 1), "gemm_ms": round(g["ms"], 3),
                       "gemm_launches": g["launches"], "int8_peak_tops": INT8_PEAK_TOPS,
                       "mfma_frac": round(tops / INT8_PEAK_TOPS, 4),
                       "valu_fold_ceiling_tops": round(fold_ceiling, 1),
                       "frac_of_fold_ceiling": round(tops / fold_ceiling, 4), "fold_valu_ops": 3,
-                      "frac_of_4op_fold_ceiling": round(tops / fold4_ceiling, 4),
                       "all_kernels_ms": round(sum(v["ms"] for v in pprof.values()), 3)}
         log(f"prefill projections: {tops:.1f} TOP/s over {g['launches']} launches "
             f"({tops / INT8_PEAK_TOPS:.3f} of the int8 peak, {tops / fold_ceiling:.3f} of the fold ceiling)")

@@ -23,11 +23,11 @@ namespace cm {
 // value 1.5 * 2^23 + dot (ulp 1 in [2^23, 2^24)), and fma(f, w, -(1.5 * 2^23) w) = round(f w -
 // 1.5 * 2^23 w) = round(dot w) exactly (the FMA rounds once, -(1.5 * 2^23) w is exact for every
 // finite f16 w: 13 significant bits, no overflow); then * xs, then +.  The scale is widened to f32
-// when it is staged: v_fma_f32 on f32 registers, v_mul_f32 and v_add_f32 fold 1024 outputs in 150
-// clocks of a SIMD (four waves), where v_fma_mix_f32 on the f16 scale takes 197.  An infinite w
-// is the one value the FMA form does not give (dot * w = +-inf, or NaN at dot = 0): a workgroup
-// that has staged one runs its remaining steps in the plain form (conversion, product), which is
-// the same for every other value.
+// when it is staged: v_fma_f32 on f32 registers, v_mul_f32 and v_add_f32 alone fold 1024 outputs
+// in 108 clocks of a SIMD (45 ns, and 51 ns with the whole device at it; two or four waves), the plain
+// form with its conversion in 141.  An infinite w is the one value the FMA form does not give
+// (dot * w = +-inf, or NaN at dot = 0): a workgroup that has staged one runs its remaining steps in
+// the plain form (conversion, product), which is the same for every other value.
 // Workgroup: 2 (rows) x 2 (tokens) waves of M x M each.  Operands move in steps of SB blocks: 16-byte
 // global loads into registers one step ahead, at the next step's start into the other half of a
 // double-buffered LDS tile [16-byte chunk][row] (planes padded so that the chunks of a row's load
@@ -35,8 +35,10 @@ namespace cm {
 // Tiles are dealt so that each XCD (workgroup id mod 8) runs a contiguous range of tiles, token
 // tiles innermost: a row tile's weights are read once per XCD and re-read from its L2.
 // Two forms.  M = 32, SB = 4 (64 x 64 tiles, four workgroups per CU) where there are tiles for the
-// device; its fold runs at about 160 clocks per 1024 outputs, and the clock falls to 1.8-2.1 GHz
-// under matrix cores, LDS and VALU together, so it is bound by power as much as by issue.  M = 16,
+// device; [128256 x 3072] x 512 takes 135 ns per 1024 outputs, block and SIMD, 2.7 times the bare
+// fold: the matrix instruction, the LDS reads of the operands and scales and the fold share the
+// issue slots, and the clock falls to 1.8-2.1 GHz under them, so it is bound by power as much as
+// by issue.  M = 16,
 // SB = 8, PIPE (32 x 32 tiles, 4 outputs per lane, each block's operands read and products issued
 // during the previous block's fold) for short prompts and narrow matrices, where a wave has its
 // SIMD to itself and its own latency per block sets the time.  Measured (us, the previous
